@@ -585,6 +585,57 @@ struct LayElems<void, D> {
   static constexpr int value = D::elems;
 };
 
+// Twiddles and butterfly j of one Stockham pass (accumulated size Ns, radix R) on the
+// R values w: w_r *= W_{Ns R}^{r (j mod Ns)}, then DFT_R.  PTAB: tw is the pass's
+// per-pass table (see BlockFFT2), else the W_L^e table.
+template <typename T, int L, int DIR, int Ns, int R, bool PTAB>
+__device__ __forceinline__ void butterfly(cx<T>* w, const __attribute__((address_space(1))) cx<T>* tw, unsigned j) {
+  if constexpr (Ns > 1) {
+    auto twiddle = [&](unsigned e) -> cx<T> {
+      cx<T> x;
+      x.x = tw[e].x;
+      x.y = DIR > 0 ? -tw[e].y : tw[e].y;
+      return x;
+    };
+    const unsigned k = j % Ns;
+    constexpr unsigned step = L / (Ns * R);
+    if constexpr (PTAB) {
+      static_assert(sizeof(T) == 4 && R % 2 == 0, "per-pass tables: FP32, even radix");
+      // row k of this pass's table, 16-byte aligned (rows of R entries); entries
+      // r = 1 .. R-1 at row[r-1], loaded two at a time
+      typedef float f4 __attribute__((ext_vector_type(4)));
+      const __attribute__((address_space(1))) f4* row =
+          (const __attribute__((address_space(1))) f4*)(tw + k * (unsigned)R);
+#pragma unroll
+      for (int q = 0; q < R / 2; ++q) {
+        const f4 two = row[q];
+        w[2 * q + 1] = cmul(w[2 * q + 1], mk(T(two.x), T(two.y)));
+        if (2 * q + 2 < R) w[2 * q + 2] = cmul(w[2 * q + 2], mk(T(two.z), T(two.w)));
+      }
+    } else if constexpr (sizeof(T) == 8) {
+      // FP64: one table load per butterfly, the other powers by repeated
+      // multiplication (w^(r+1) = w^r w, below 22 ulp at R = 24).  Each saved
+      // load is a full vector-memory instruction through the texture path; the
+      // chain costs four FMA-class operations and keeps two powers live.
+      // Loading every power instead made the 768-point FP64 row kernel 12 %
+      // slower (6.39 against 5.72 ms per 512^3 launch; column passes unchanged).
+      const cx<T> w1 = twiddle(k * step);
+      cx<T> wr = w1;
+      w[1] = cmul_fixed(w[1], w1);
+#pragma unroll
+      for (int r = 2; r < R; ++r) {
+        wr = cmul_fixed(wr, w1);
+        w[r] = cmul_fixed(w[r], wr);
+      }
+    } else {
+      // FP32 loads every power: a chain's error would rival the transform's own
+#pragma unroll
+      for (int r = 1; r < R; ++r) w[r] = cmul(w[r], twiddle(r * k * step));
+    }
+  }
+  DFT<R, DIR, T>::run(w);
+}
+
 // MIDW / MIDH: bit P set = middle pass P uses MAP_WAVE / MAP_HALF instead of
 // MAP_STD.  PADE: pad period of the swizzled layout in elements (0: one 16-byte
 // complex per slot).  LSEL: per-exchange layouts (void: ExLayout for every
@@ -643,13 +694,6 @@ struct BlockFFT2 {
   // wait counter
   using twptr = const __attribute__((address_space(1))) cx<T>*;
 
-  __device__ __forceinline__ static cx<T> twiddle(twptr tw, unsigned e) {
-    cx<T> w;
-    w.x = tw[e].x;
-    w.y = DIR > 0 ? -tw[e].y : tw[e].y;
-    return w;
-  }
-
   template <int MAP, int Ns, int R>
   __device__ __forceinline__ static void butterflies(cx<T>* v, int t_in, const cx<T>* __restrict__ tw_in) {
     static_assert(E % R == 0, "radix must divide E");
@@ -663,47 +707,9 @@ struct BlockFFT2 {
     __builtin_assume(t < (unsigned)NT);
 #pragma unroll
     for (int b = 0; b < E / R; ++b) {
-      cx<T>* w = v + b * R;
-      if (Ns > 1) {
-        unsigned s, j;
-        bmap<MAP, TS, NT, L, R, G>(t, b, s, j);
-        const unsigned k = j % Ns;
-        constexpr unsigned step = L / (Ns * R);
-        if constexpr (PTAB) {
-          static_assert(sizeof(T) == 4 && R % 2 == 0, "per-pass tables: FP32, even radix");
-          // row k of this pass's table, 16-byte aligned (rows of R entries); entries
-          // r = 1 .. R-1 at row[r-1], loaded two at a time
-          typedef float f4 __attribute__((ext_vector_type(4)));
-          const __attribute__((address_space(1))) f4* row =
-              (const __attribute__((address_space(1))) f4*)(tw + k * (unsigned)R);
-#pragma unroll
-          for (int q = 0; q < R / 2; ++q) {
-            const f4 two = row[q];
-            w[2 * q + 1] = cmul(w[2 * q + 1], mk(T(two.x), T(two.y)));
-            if (2 * q + 2 < R) w[2 * q + 2] = cmul(w[2 * q + 2], mk(T(two.z), T(two.w)));
-          }
-        } else if (sizeof(T) == 8) {
-          // FP64: one table load per butterfly, the other powers by repeated
-          // multiplication (w^(r+1) = w^r w, below 22 ulp at R = 24).  Each saved
-          // load is a full vector-memory instruction through the texture path; the
-          // chain costs four FMA-class operations and keeps two powers live.
-          // Loading every power instead made the 768-point FP64 row kernel 12 %
-          // slower (6.39 against 5.72 ms per 512^3 launch; column passes unchanged).
-          const cx<T> w1 = twiddle(tw, k * step);
-          cx<T> wr = w1;
-          w[1] = cmul_fixed(w[1], w1);
-#pragma unroll
-          for (int r = 2; r < R; ++r) {
-            wr = cmul_fixed(wr, w1);
-            w[r] = cmul_fixed(w[r], wr);
-          }
-        } else {
-          // FP32 loads every power: a chain's error would rival the transform's own
-#pragma unroll
-          for (int r = 1; r < R; ++r) w[r] = cmul(w[r], twiddle(tw, r * k * step));
-        }
-      }
-      DFT<R, DIR, T>::run(w);
+      unsigned s = 0, j = 0;
+      if (Ns > 1) bmap<MAP, TS, NT, L, R, G>(t, b, s, j);
+      butterfly<T, L, DIR, Ns, R, PTAB>(v + b * R, tw, j);
     }
   }
 

@@ -10,7 +10,9 @@
 //       K5 col  forward axis 0, rows M -> N kept  => B_hat on the N-grid
 //       K6 k-space: i k.B_hat, Leray projection, SmoothCutoff viscosity, fused with
 //               the RK stage update
-//   2D: K1 col axis 0, K2 row axis 1, K3 col axis 0, K4 k-space.
+//   2D: K1 row axis 1, K2 column stage (azb_stage.hpp): forward axis 0, k-space with the
+//       stage update, inverse axis 0 of the new stage value; or, where separate passes are
+//       faster, K1 col axis 0, K2 row axis 1, K3 col axis 0, K4 k-space.
 //
 // Reference behaviour restated here: copy_to_padded (copy_to_padded_functions.hpp:
 // 11-63), the FFTW/cuFFT c2r convention (complex passes on the leading axes, then
@@ -41,7 +43,7 @@ struct DevState {
 };
 
 enum ColMode { COL_PAD_IN = 0, COL_TRUNC_OUT = 1, COL_FULL = 2 };
-enum KMode { K_DUDT = 0, K_RK1 = 1, K_RK2 = 2, K_RK3 = 3 };
+enum KMode { K_DUDT = 0, K_RK1 = 1, K_RK2 = 2, K_RK3 = 3, K_LEAD = 4 };
 
 // E (complex values per thread) and radix plan per transform length
 template <int L>
@@ -198,16 +200,32 @@ __global__ __launch_bounds__(TS * L / LenPlan<L>::E, (sizeof(T) == 4 ? 4 : (L ==
 // separated into the two half spectra; only k <= N/2 is written.
 // ---------------------------------------------------------------------------
 struct RowArgs {
-  const void* in;   // [c][line][ls]: N/2+1 modes per line
+  const void* in;   // [c][line][ls] (2D: or column blocks): N/2+1 modes per line
   void* out;        // [m][line][ls]
   long nlines;      // lines per component (M for 2D, M*M for 3D)
-  long ls;          // line stride (elements, >= N/2+1)
+  long ls;          // line stride (elements): >= N/2+1, or bw
+  int bw;           // 2D: width of column blocks (a power of two), [c][k / bw][line][k % bw]; 0: plain lines
   long in_ss, out_ss;  // sample strides (elements)
   double norm;      // 1 / (N^{d/2} M^{d/2})
   const void* tw;
   DevState* st;
   int slot;         // umax slot
+  int begin;        // first kernel of a step of the device-driven loop (see row_idle)
 };
+
+// Whether this workgroup's sample sits the launch out.  In the first kernel of a loop step
+// every workgroup decides from the sample's time, which no kernel of the previous step
+// still writes, and the sample's first workgroup records the decision and the step's clamp
+// for the kernels that follow (step_prologue_loop's work without its launch).
+__device__ __forceinline__ bool row_idle(const RowArgs& a, DevState* st, bool first) {
+  if (!a.begin) return st->done != 0;
+  const bool go = st->time < st->t_end;
+  if (first && threadIdx.x == 0) {
+    st->done = go ? 0 : 1;
+    if (go) st->max_dt = fmin(st->t_end - st->time, st->max_dt_visc);
+  }
+  return !go;
+}
 
 template <typename T>
 __device__ __forceinline__ double wave_max(double v) {
@@ -263,9 +281,89 @@ __device__ __forceinline__ double sv_eval(double k, double eps, double s2, doubl
   return -eps * kp * qk;
 }
 
-__device__ __forceinline__ double2 cmuli(double k, double2 b) {
-  // complex_t(0, k) * b
-  return make_double2(0.0 * b.x - k * b.y, 0.0 * b.y + k * b.x);
+// One mode's wavevector, |k|^2 and Leray projector 1 - k k^T / |k|^2 (symmetric:
+// P11, P12, P22 in 2D; P11, P21, P22, P31, P32, P33 in 3D).
+constexpr double kTwoPi = 2.0 * 3.14159265358979323846;
+template <int DIM>
+struct ModeGeom {
+  double k[3], P[6], absk2;
+  // 2D: signed mode number i of axis 0, kk of the last axis, inv = 1 / |k|^2 from the
+  // caller's table, or computed here
+  __device__ __forceinline__ void set2(int i, int kk, double inv, bool have_inv) {
+    const double k1 = kTwoPi * i, k2 = kTwoPi * kk;
+    absk2 = k1 * k1 + k2 * k2;
+    if (!have_inv) inv = 1.0 / absk2;
+    const double k11 = k1 * k1 * inv, k12 = k1 * k2 * inv, k22 = k2 * k2 * inv;
+    k[0] = k1; k[1] = k2;
+    P[0] = 1.0 - k11; P[1] = 0.0 - k12; P[2] = 1.0 - k22;
+  }
+  __device__ __forceinline__ ModeGeom(int i, int kk, double inv) { set2(i, kk, inv, true); }
+  // signed mode numbers i, j of the full axes (2D: i only), kk of the last
+  __device__ __forceinline__ ModeGeom(int i, int j, int kk) {
+    if (DIM == 2) {
+      set2(i, kk, 0.0, false);
+      return;
+    }
+    const double k1 = kTwoPi * i, k2 = kTwoPi * j, k3 = kTwoPi * kk;
+    absk2 = k1 * k1 + k2 * k2 + k3 * k3;
+    const double inv = 1.0 / absk2;
+    const double k11 = k1 * k1 * inv, k12 = k1 * k2 * inv, k13 = k1 * k3 * inv;
+    const double k22 = k2 * k2 * inv, k23 = k2 * k3 * inv, k33 = k3 * k3 * inv;
+    k[0] = k1; k[1] = k2; k[2] = k3;
+    P[0] = 1.0 - k11; P[1] = 0.0 - k12; P[2] = 1.0 - k22;
+    P[3] = 0.0 - k13; P[4] = 0.0 - k23; P[5] = 1.0 - k33;
+  }
+};
+
+// b = k . B for one half (real or imaginary parts) of the products B_m at a mode: ik.B_hat
+// maps Re B to the imaginary part of b and -Im B to its real part, so the two halves never
+// meet and a caller may hold one at a time.
+template <int DIM>
+__device__ __forceinline__ void kspace_dot(const ModeGeom<DIM>& g, const double* B, double* b) {
+  if (DIM == 2) {
+    const double t1 = g.k[0] * B[0], t2 = g.k[1] * B[1];
+    const double t3 = g.k[0] * B[1], t4 = g.k[1] * B[2];
+    b[0] = t1 + t2;
+    b[1] = t3 + t4;
+  } else {
+    {
+      const double x = g.k[0] * B[0], y = g.k[1] * B[1], z = g.k[2] * B[3];
+      b[0] = x + y + z;
+    }
+    {
+      const double x = g.k[0] * B[1], y = g.k[1] * B[2], z = g.k[2] * B[4];
+      b[1] = x + y + z;
+    }
+    {
+      const double x = g.k[0] * B[3], y = g.k[1] * B[4], z = g.k[2] * B[5];
+      b[2] = x + y + z;
+    }
+  }
+}
+
+// L = P b, the Leray projection of one half
+template <int DIM>
+__device__ __forceinline__ void kspace_project(const ModeGeom<DIM>& g, const double* b, double* L) {
+  if (DIM == 2) {
+    L[0] = g.P[0] * b[0] + g.P[1] * b[1];
+    L[1] = g.P[1] * b[0] + g.P[2] * b[1];
+  } else {
+    L[0] = g.P[0] * b[0] + g.P[1] * b[1] + g.P[3] * b[2];
+    L[1] = g.P[1] * b[0] + g.P[2] * b[1] + g.P[4] * b[2];
+    L[2] = g.P[3] * b[0] + g.P[4] * b[1] + g.P[5] * b[2];
+  }
+}
+
+// One real component of du/dt = -L + nu u (0 at k = 0) and of the RK stage value made
+// from it: u the stage input, w the RK base state (stages 2 and 3).
+__device__ __forceinline__ double stage_value(int mode, double absk2, double L, double nu, double u, double w,
+                                              double dt) {
+  const double d = absk2 == 0 ? 0.0 : -L + nu * u;
+  if (mode == K_DUDT) return d;
+  const double tmp = 1.0 * u + dt * d;
+  if (mode == K_RK1) return tmp;
+  if (mode == K_RK2) return 0.75 * w + 0.25 * tmp;
+  return (2.0 / 3) * tmp + (1.0 / 3) * w;
 }
 
 template <typename T, int DIM>
@@ -296,7 +394,6 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
   }
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= a.nmodes) return;
-  const double twopi = 2.0 * 3.14159265358979323846;
   const int N = a.n, NH = a.nh;
   const cx<T>* bh = (const cx<T>*)a.bh + sample * (3 * (DIM - 1)) * a.bstride;
   // 32-bit index arithmetic: the supported grids have fewer than 2^27 modes per component
@@ -304,87 +401,31 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
   const int kk = (int)(ui % (unsigned)NH);
   const unsigned rest = ui / (unsigned)NH;
   const long bidx = (long)rest * a.nhp + kk;
-  auto B = [&](int m) -> double2 {
-    const cx<T> z = ntload<T>(bh + (long)m * a.bstride + bidx);
-    return make_double2((double)z.x, (double)z.y);
-  };
-  double absk2;
-  double2 L[3];
-  if (DIM == 2) {
-    const int i = (int)rest;
-    const int i_ = i >= N / 2 + 1 ? i - N : i;
-    const double k1 = twopi * i_;
-    const double k2 = twopi * kk;
-    absk2 = k1 * k1 + k2 * k2;
-    const double2 B11 = B(0), B12 = B(1), B22 = B(2);
-    const double2 t1 = cmuli(k1, B11), t2 = cmuli(k2, B12);
-    const double2 b1 = make_double2(t1.x + t2.x, t1.y + t2.y);
-    const double2 t3 = cmuli(k1, B12), t4 = cmuli(k2, B22);
-    const double2 b2 = make_double2(t3.x + t4.x, t3.y + t4.y);
-    const double inv = 1.0 / absk2;
-    const double k11 = k1 * k1 * inv, k12 = k1 * k2 * inv, k22 = k2 * k2 * inv;
-    const double c11 = 1.0 - k11, c12 = 0.0 - k12, c22 = 1.0 - k22;
-    L[0] = make_double2(c11 * b1.x + c12 * b2.x, c11 * b1.y + c12 * b2.y);
-    L[1] = make_double2(c12 * b1.x + c22 * b2.x, c12 * b1.y + c22 * b2.y);
-  } else {
-    const int j = (int)(rest % (unsigned)N);
-    const int i = (int)(rest / (unsigned)N);
-    const int i_ = i >= N / 2 + 1 ? i - N : i;
-    const int j_ = j >= N / 2 + 1 ? j - N : j;
-    const double k1 = twopi * i_, k2 = twopi * j_, k3 = twopi * kk;
-    absk2 = k1 * k1 + k2 * k2 + k3 * k3;
-    const double2 B11 = B(0), B21 = B(1), B22 = B(2), B31 = B(3), B32 = B(4), B33 = B(5);
-    double2 b[3];
-    {
-      const double2 x = cmuli(k1, B11), y = cmuli(k2, B21), z = cmuli(k3, B31);
-      b[0] = make_double2(x.x + y.x + z.x, x.y + y.y + z.y);
-    }
-    {
-      const double2 x = cmuli(k1, B21), y = cmuli(k2, B22), z = cmuli(k3, B32);
-      b[1] = make_double2(x.x + y.x + z.x, x.y + y.y + z.y);
-    }
-    {
-      const double2 x = cmuli(k1, B31), y = cmuli(k2, B32), z = cmuli(k3, B33);
-      b[2] = make_double2(x.x + y.x + z.x, x.y + y.y + z.y);
-    }
-    const double inv = 1.0 / absk2;
-    const double k11 = k1 * k1 * inv, k12 = k1 * k2 * inv, k13 = k1 * k3 * inv;
-    const double k22 = k2 * k2 * inv, k23 = k2 * k3 * inv, k33 = k3 * k3 * inv;
-    const double P[3][3] = {{1.0 - k11, 0.0 - k12, 0.0 - k13},
-                            {0.0 - k12, 1.0 - k22, 0.0 - k23},
-                            {0.0 - k13, 0.0 - k23, 1.0 - k33}};
+  const int j = DIM == 3 ? (int)(rest % (unsigned)N) : 0;
+  const int i = DIM == 3 ? (int)(rest / (unsigned)N) : (int)rest;
+  const ModeGeom<DIM> g(i >= N / 2 + 1 ? i - N : i, j >= N / 2 + 1 ? j - N : j, kk);
+  constexpr int NM = 3 * (DIM - 1);
+  double Br[NM], Bi[NM], b[DIM], Lr[DIM], Li[DIM];
 #pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      L[r] = make_double2(P[r][0] * b[0].x + P[r][1] * b[1].x + P[r][2] * b[2].x,
-                          P[r][0] * b[0].y + P[r][1] * b[1].y + P[r][2] * b[2].y);
-    }
+  for (int m = 0; m < NM; ++m) {
+    const cx<T> z = ntload<T>(bh + (long)m * a.bstride + bidx);
+    Br[m] = (double)z.x;
+    Bi[m] = -(double)z.y;
   }
-  const double nu = sv_eval(sqrt(absk2), a.eps, a.s2, a.k0);
+  kspace_dot<DIM>(g, Bi, b);
+  kspace_project<DIM>(g, b, Lr);
+  kspace_dot<DIM>(g, Br, b);
+  kspace_project<DIM>(g, b, Li);
+  const double nu = sv_eval(sqrt(g.absk2), a.eps, a.s2, a.k0);
 #pragma unroll
   for (int c = 0; c < DIM; ++c) {
     const long o = (sample * DIM + c) * a.nmodes + idx;
-    const cx<double> uu = ntload<double>(a.u_in + o);
-    const double2 u = make_double2(uu.x, uu.y);
-    double2 d = absk2 == 0 ? make_double2(0.0, 0.0)
-                           : make_double2(-L[c].x + nu * u.x, -L[c].y + nu * u.y);
-    double2 r;
-    if (a.mode == K_DUDT) {
-      r = d;
-    } else if (a.mode == K_RK1) {
-      r = make_double2(1.0 * u.x + dt * d.x, 1.0 * u.y + dt * d.y);
-    } else {
-      const double2 tmp = make_double2(1.0 * u.x + dt * d.x, 1.0 * u.y + dt * d.y);
-      const cx<double> ww = ntload<double>(a.u0 + o);
-      const double2 w = make_double2(ww.x, ww.y);
-      if (a.mode == K_RK2) {
-        r = make_double2(0.75 * w.x + 0.25 * tmp.x, 0.75 * w.y + 0.25 * tmp.y);
-      } else {
-        r = make_double2((2.0 / 3) * tmp.x + (1.0 / 3) * w.x, (2.0 / 3) * tmp.y + (1.0 / 3) * w.y);
-      }
-    }
+    const cx<double> u = ntload<double>(a.u_in + o);
+    cx<double> w = mk(0.0, 0.0);
+    if (a.mode == K_RK2 || a.mode == K_RK3) w = ntload<double>(a.u0 + o);
     vec2_t<double> rv;
-    rv.x = r.x;
-    rv.y = r.y;
+    rv.x = stage_value(a.mode, g.absk2, Lr[c], nu, u.x, w.x, dt);
+    rv.y = stage_value(a.mode, g.absk2, Li[c], nu, u.y, w.y, dt);
     __builtin_nontemporal_store(rv, (vec2_t<double>*)(a.out + o));
   }
 }
@@ -504,6 +545,22 @@ namespace azb {
 //              values a thread needs for separation come over lane permutes, and
 //              the k <= N/2 outputs leave as contiguous 16-byte stores.
 // ---------------------------------------------------------------------------
+// Where mode k of a line lies relative to the line's base: plain (contiguous) or in column
+// blocks of bw modes with M lines between a block and the next (the 2D kernels).
+struct PlainCols {
+  __device__ __forceinline__ unsigned at(unsigned k) const { return k; }
+};
+struct BlockCols {
+  unsigned sh, mask, stride;
+  // bw = 0: plain lines of stride ls
+  __device__ __forceinline__ BlockCols(int bw, long ls, long nlines)
+      : sh(bw ? 31u - (unsigned)__clz(bw) : 31u), mask(bw ? (unsigned)bw - 1 : 0x7fffffffu),
+        stride((unsigned)nlines * (unsigned)ls) {}
+  __device__ __forceinline__ unsigned at(unsigned k) const { return (k >> sh) * stride + (k & mask); }
+  // elements of one component
+  __device__ __forceinline__ long comp(int nmodes) const { return (long)(((unsigned)nmodes + mask) >> sh) * stride; }
+};
+
 // Packed first inverse pass of a row kernel, from HBM: radix R (12 or 24) with one
 // butterfly per thread, butterfly j (< NB = L/R) of a sequence X + iY at positions
 // j + NB r, X and Y the half spectra (N/2 + 1 modes) of two real lines.  Positions
@@ -511,26 +568,28 @@ namespace azb {
 // from L - N/2 = (2R/3) NB read the conjugates at k = L - pos (r >= 2R/3), the rest
 // are the zero padding; the k = 0 entry drops Im as the reference's c2r does.  Ends
 // with the radix-R DFT.
-template <typename T, int NB, int R = 12>
+template <typename T, int NB, int R = 12, class Cols = PlainCols>
 __device__ __forceinline__ void row_first_pass(cx<T>* v, const cx<T>* __restrict__ px,
-                                               const cx<T>* __restrict__ py, unsigned j) {
+                                               const cx<T>* __restrict__ py, unsigned j, Cols cols = Cols{}) {
   static_assert(R % 3 == 0, "N/2 = L/3 must fall on a butterfly row");
   constexpr int R3 = R / 3;
   const bool j0 = j == 0;
+  // NB is a multiple of every block width, so a step of NB modes is a constant stride
+  const unsigned at = cols.at(j), mat = cols.at(NB - j), step = cols.at(NB);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (r < R3) {
-      const cx<T> X0 = px[j + NB * r], Y0 = py[j + NB * r];
+      const cx<T> X0 = px[at + step * r], Y0 = py[at + step * r];
       v[r] = mk(X0.x - Y0.y, X0.y + Y0.x);
       if (r == 0 && j0) v[r] = mk(X0.x, Y0.x);
     } else if (r >= 2 * R3) {
-      const unsigned kk = NB * (R - r) - j;
+      const unsigned kk = mat + step * (R - 1 - r);  // mode NB (R - r) - j
       const cx<T> X0 = px[kk], Y0 = py[kk];
       v[r] = mk(X0.x + Y0.y, Y0.x - X0.y);
     } else {
       v[r] = mk(T(0), T(0));
       if (r == R3 && j0) {
-        const cx<T> X0 = px[R3 * NB], Y0 = py[R3 * NB];
+        const cx<T> X0 = px[R3 * step], Y0 = py[R3 * step];
         v[r] = mk(X0.x - Y0.y, X0.y + Y0.x);
       }
     }
@@ -546,9 +605,10 @@ __device__ __forceinline__ void row_first_pass(cx<T>* v, const cx<T>* __restrict
 // butterfly NB - j (for j = 0: index R - r of this lane).  Stores A[k], B[k] for the
 // k <= N/2 = (R/3) NB this lane owns (r < R/3, and r = R/3 for j = 0) as contiguous
 // non-temporal stores.
-template <typename T, int NB, int R = 12>
+template <typename T, int NB, int R = 12, class Cols = PlainCols>
 __device__ __forceinline__ void row_separate_store(const cx<T>* v, unsigned lane, unsigned j, vec2_t<T>* oa,
-                                                   vec2_t<T>* ob) {
+                                                   vec2_t<T>* ob, Cols cols = Cols{}) {
+  const unsigned at = cols.at(j), step = cols.at(NB);
   constexpr int R3 = R / 3;
   // butterfly j of a sequence in lane j of its wave (or half-wave)
   static_assert(64 % NB == 0, "a sequence's butterflies within one wave");
@@ -577,9 +637,9 @@ __device__ __forceinline__ void row_separate_store(const cx<T>* v, unsigned lane
     } else {
       if (j0) zm = f[r - 1];
     }
-    emit(j + NB * r, v[r], zm);
+    emit(at + step * r, v[r], zm);
   }
-  if (j0) emit(R3 * NB, v[R3], f[R3 - 1]);
+  if (j0) emit(R3 * step, v[R3], f[R3 - 1]);
 }
 
 template <int L>
@@ -615,7 +675,7 @@ __global__ __launch_bounds__(P * L / 4) __attribute__((amdgpu_waves_per_eu(sizeo
   const long bps = a.nlines / (2 * P);  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (st->done) return;
+  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
 
   const int t = threadIdx.x;
   const long line0 = (blockIdx.x % bps) * (2 * P);
@@ -764,7 +824,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const long bps = a.nlines / (2 * P);  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (st->done) return;
+  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
 
   const int t = threadIdx.x;
   const long line0 = (blockIdx.x % bps) * (2 * P);
@@ -910,7 +970,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const long bps = a.nlines / 2;  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (st->done) return;
+  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
 
   const int t = threadIdx.x;
   const long la = (blockIdx.x % bps) * 2, lb = la + 1;
@@ -1017,16 +1077,19 @@ __global__ __launch_bounds__((Row2Cfg<T, L>::NT)) void euler_row2_kernel(RowArgs
   __shared__ T X[C::XWORDS];
   __shared__ double red[NT / 64];
   const long bps = a.nlines / (2 * P);  // workgroups per sample
-  const long sample = blockIdx.x / bps;
+  const unsigned blk = xcd_contiguous(blockIdx.x, gridDim.x);
+  const long sample = blk / bps;
   DevState* st = a.st + sample;
-  if (st->done) return;
+  if (row_idle(a, st, blk % bps == 0)) return;
 
   const int t = threadIdx.x;
-  const long line0 = (blockIdx.x % bps) * (2 * P);
+  const long line0 = (blk % bps) * (2 * P);
   const cx<T>* __restrict__ in = (const cx<T>*)a.in + sample * a.in_ss;
   cx<T>* __restrict__ out = (cx<T>*)a.out + sample * a.out_ss;
   const cx<T>* __restrict__ tw = (const cx<T>*)a.tw;
   const T nrm = T(a.norm);
+  const BlockCols cols(a.bw, a.ls, a.nlines);
+  const long cs = cols.comp(L / 3 + 1);  // component stride (N/2 + 1 = L/3 + 1 modes)
 
   cx<T> v[12];
   {
@@ -1035,7 +1098,7 @@ __global__ __launch_bounds__((Row2Cfg<T, L>::NT)) void euler_row2_kernel(RowArgs
     if (tt < (unsigned)(TSI * NB)) {
       const unsigned s = tt / NB, j = tt % NB;  // sequence s: u1 + i u2 of line line0 + s
       const long l = line0 + s;
-      row_first_pass<T, NB>(v, in + l * a.ls, in + (a.nlines + l) * a.ls, j);
+      row_first_pass<T, NB, 12>(v, in + l * a.ls, in + cs + l * a.ls, j, cols);
       // Stockham pass-0 outputs of butterfly j sit at positions 12 j + r
 #pragma unroll
       for (int r = 0; r < 12; ++r) {
@@ -1069,8 +1132,8 @@ __global__ __launch_bounds__((Row2Cfg<T, L>::NT)) void euler_row2_kernel(RowArgs
     bmap<MAPL, TSF, NT, L, 12, 3>(tt, 0, s, j);
     const unsigned pair = s / 3, m = s % 3;
     const long la = line0 + 2 * pair, lb = la + 1;
-    row_separate_store<T, NB>(w, tt & 63, j, (vec2_t<T>*)(out + ((long)m * a.nlines + la) * a.ls),
-                              (vec2_t<T>*)(out + ((long)m * a.nlines + lb) * a.ls));
+    row_separate_store<T, NB, 12>(w, tt & 63, j, (vec2_t<T>*)(out + m * cs + la * a.ls),
+                              (vec2_t<T>*)(out + m * cs + lb * a.ls), cols);
   }
 
   lmax = wave_max<T>(lmax);
@@ -1123,16 +1186,19 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void e
   __shared__ T X[XWORDS];
   __shared__ double red[NT / 64];
   const long bps = a.nlines / 2;  // workgroups per sample
-  const long sample = blockIdx.x / bps;
+  const unsigned blk = xcd_contiguous(blockIdx.x, gridDim.x);
+  const long sample = blk / bps;
   DevState* st = a.st + sample;
-  if (st->done) return;
+  if (row_idle(a, st, blk % bps == 0)) return;
 
   const int t = threadIdx.x;
-  const long la = (blockIdx.x % bps) * 2, lb = la + 1;
+  const long la = (blk % bps) * 2, lb = la + 1;
   const cx<T>* __restrict__ in = (const cx<T>*)a.in + sample * a.in_ss;
   cx<T>* __restrict__ out = (cx<T>*)a.out + sample * a.out_ss;
   const cx<T>* __restrict__ tw = (const cx<T>*)a.tw;
   const T nrm = T(a.norm);
+  const BlockCols cols(a.bw, a.ls, a.nlines);
+  const long cs = cols.comp(L / 3 + 1);  // component stride (N/2 + 1 = L/3 + 1 modes)
 
   cx<T> v[24];
   {
@@ -1141,7 +1207,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void e
     if (tt < (unsigned)(2 * NB)) {
       const unsigned s = tt / NB, j = tt % NB;  // sequence s: u1 + i u2 of line la + s
       const long l = la + s;
-      row_first_pass<T, NB, 24>(v, in + l * a.ls, in + (a.nlines + l) * a.ls, j);
+      row_first_pass<T, NB, 24>(v, in + l * a.ls, in + cs + l * a.ls, j, cols);
       // Stockham pass-0 outputs of butterfly j sit at positions 24 j + r
 #pragma unroll
       for (int r = 0; r < 24; ++r) {
@@ -1173,8 +1239,8 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void e
     unsigned tt = t;
     asm volatile("" : "+v"(tt));
     const unsigned m = tt / NB, j = tt % NB;
-    row_separate_store<T, NB, 24>(w, tt & 63, j, (vec2_t<T>*)(out + ((long)m * a.nlines + la) * a.ls),
-                                  (vec2_t<T>*)(out + ((long)m * a.nlines + lb) * a.ls));
+    row_separate_store<T, NB, 24>(w, tt & 63, j, (vec2_t<T>*)(out + m * cs + la * a.ls),
+                                  (vec2_t<T>*)(out + m * cs + lb * a.ls), cols);
   }
 
   lmax = wave_max<T>(lmax);
@@ -1238,18 +1304,21 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   __shared__ T X[XWORDS];
   __shared__ double red[NT / 64];
   const long bps = a.nlines / (2 * P);  // workgroups per sample
-  const long sample = blockIdx.x / bps;
+  const unsigned blk = xcd_contiguous(blockIdx.x, gridDim.x);
+  const long sample = blk / bps;
   DevState* st = a.st + sample;
-  if (st->done) return;
+  if (row_idle(a, st, blk % bps == 0)) return;
 
   const int t = threadIdx.x;
-  const long line0 = (blockIdx.x % bps) * (2 * P);
+  const long line0 = (blk % bps) * (2 * P);
   const cx<T>* __restrict__ in = (const cx<T>*)a.in + sample * a.in_ss;
   cx<T>* __restrict__ out = (cx<T>*)a.out + sample * a.out_ss;
   const cx<T>* __restrict__ tw = (const cx<T>*)a.tw;
   const cx<T>* twi = PT ? tw + Row8Cfg<float, 768>::TW_INV : tw;
   const cx<T>* twf = PT ? tw + Row8Cfg<float, 768>::TW_FWD : tw;
   const T nrm = T(a.norm);
+  const BlockCols cols(a.bw, a.ls, a.nlines);
+  const long cs = cols.comp(L / 3 + 1);  // component stride (N/2 + 1 = L/3 + 1 modes)
 
   cx<T> v[24];
   if constexpr (!SPI) {
@@ -1258,7 +1327,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     if (tt < (unsigned)(2 * P * NB)) {
       const unsigned s = tt / NB, j = tt % NB;  // sequence s: u1 + i u2 of line line0 + s
       const long l = line0 + s;
-      row_first_pass<T, NB, 24>(v, in + l * a.ls, in + (a.nlines + l) * a.ls, j);
+      row_first_pass<T, NB, 24>(v, in + l * a.ls, in + cs + l * a.ls, j, cols);
       // Stockham pass-0 outputs of butterfly j sit at positions 24 j + r
 #pragma unroll
       for (int r = 0; r < 24; ++r) {
@@ -1279,7 +1348,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     const unsigned s0 = tt / NB, j0 = tt % NB;
     if (writer) {
       const long l = line0 + s0;
-      row_first_pass<T, NB, 24>(v, in + l * a.ls, in + (a.nlines + l) * a.ls, j0);
+      row_first_pass<T, NB, 24>(v, in + l * a.ls, in + cs + l * a.ls, j0, cols);
     }
     cx<T> x[16];
 #pragma unroll
@@ -1336,8 +1405,8 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     const unsigned s = tt / NB, j = tt % NB;
     const unsigned pair = s / 3, m = s % 3;
     const long la = line0 + 2 * pair, lb = la + 1;
-    row_separate_store<T, NB, 24>(w, tt & 63, j, (vec2_t<T>*)(out + ((long)m * a.nlines + la) * a.ls),
-                                  (vec2_t<T>*)(out + ((long)m * a.nlines + lb) * a.ls));
+    row_separate_store<T, NB, 24>(w, tt & 63, j, (vec2_t<T>*)(out + m * cs + la * a.ls),
+                                  (vec2_t<T>*)(out + m * cs + lb * a.ls), cols);
   }
 
   lmax = wave_max<T>(lmax);
@@ -1407,7 +1476,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   const long bps = a.nlines / (2 * P);  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (st->done) return;
+  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
 
   const int t = threadIdx.x;
   const long line0 = (blockIdx.x % bps) * (2 * P);

@@ -244,6 +244,7 @@ struct azb_solver {
   void* Z = nullptr;  // S1
   double2* u1 = nullptr;
   double2* u2 = nullptr;
+  double2* modes = nullptr;  // 2D: the column stage's mode table
   DevState* st = nullptr;
   void* tw = nullptr;
   size_t bytes = 0;
@@ -255,6 +256,7 @@ struct azb_solver {
   int pdiv = 1;
   // radix plan per column-pass family (ColPlan index; the row and k-space entries are 0)
   int plan[AZB_PROF_FAMILIES] = {0, 0, 0, 0, 0, 0};
+  StageShape stage{0, 0};  // 2D column stage; width 0: separate passes
   DevState* probe_host = nullptr;  // pinned mirror of the device state (non-blocking probes)
   hipEvent_t probe_ev = nullptr;
   // per-kernel-family hipEvent timing (off unless enabled)
@@ -299,8 +301,8 @@ struct ProfScope {
 };
 
 template <typename T>
-int enqueue_rhs_T(azb_solver* s, const double2* u_in, const double2* u0, double2* out, int kmode,
-                  int slot, double C) {
+int enqueue_rhs_3d(azb_solver* s, const double2* u_in, const double2* u0, double2* out, int kmode,
+                   int slot, double C) {
   const int N = s->N, M = s->M, nh = s->nh;
   const long S = s->S;
   const long hp = s->nhp;  // padded last-axis stride of every intermediate
@@ -316,97 +318,58 @@ int enqueue_rhs_T(azb_solver* s, const double2* u_in, const double2* u0, double2
   r.st = s->st;
   r.slot = slot;
   r.ls = hp;
-  r.norm = 1.0 / (std::pow(std::sqrt((double)N), s->dim) * std::pow(std::sqrt((double)M), s->dim));
-  if (s->dim == 3) {
-    // K1: inverse along axis 0, N -> M rows; state [c][i][j][k] -> X[c][i'][j][hp]
-    c.in = u_in; c.out = s->X; c.nq = N;
-    c.in_qs = nh; c.out_qs = hp;
-    c.in_rs = (long)N * nh; c.out_rs = (long)N * hp;
-    c.in_bs = (long)N * N * nh; c.out_bs = (long)M * N * hp;
-    c.bps = 3;
-    {
-      ProfScope p(s, AZB_PROF_INV_AX0);
-      if ((rc = launch_col<double, T, T, +1, COL_PAD_IN>(M, c, 3L * S, st, s->tsdiv[AZB_PROF_INV_AX0], s->plan[AZB_PROF_INV_AX0]))) return rc;
-    }
-    // K2: inverse along axis 1; X[c][i'][j][hp] -> Y[c][i'][j'][hp]
-    c.in = s->X; c.out = s->Y; c.nq = 1;
-    c.in_qs = 0; c.out_qs = 0;
-    c.in_rs = hp; c.out_rs = hp;
-    c.in_bs = (long)N * hp; c.out_bs = (long)M * hp;
-    c.bps = 3 * M;
-    {
-      ProfScope p(s, AZB_PROF_INV_AX1);
-      if ((rc = launch_col<T, T, T, +1, COL_PAD_IN>(M, c, 3L * M * S, st, s->tsdiv[AZB_PROF_INV_AX1], s->plan[AZB_PROF_INV_AX1]))) return rc;
-    }
-    // K3: last axis c2r, products, max, r2c; Y[c][line][hp] -> Z[m][line][hp]
-    r.in = s->Y; r.out = s->Z; r.nlines = (long)M * M;
-    r.in_ss = 3L * M * M * hp; r.out_ss = 6L * M * M * hp;
-    {
-      ProfScope p(s, AZB_PROF_ROW);
-      if ((rc = launch_row<T, 3>(M, r, S, st, s->pdiv))) return rc;
-    }
-    // K4: forward along axis 1, M -> N rows; Z[m][i'][j'][hp] -> X[m][i'][j][hp]
-    c.in = s->Z; c.out = s->X; c.nq = 1;
-    c.in_qs = 0; c.out_qs = 0;
-    c.in_rs = hp; c.out_rs = hp;
-    c.in_bs = (long)M * hp; c.out_bs = (long)N * hp;
-    c.bps = 6 * M;
-    {
-      ProfScope p(s, AZB_PROF_FWD_AX1);
-      if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 6L * M * S, st, s->tsdiv[AZB_PROF_FWD_AX1], s->plan[AZB_PROF_FWD_AX1]))) return rc;
-    }
-    // K5: forward along axis 0; X[m][i'][j][hp] -> Y[m][i][j][hp] (B_hat on the N-grid)
-    c.in = s->X; c.out = s->Y; c.nq = N;
-    c.in_qs = hp; c.out_qs = hp;
-    c.in_rs = (long)N * hp; c.out_rs = (long)N * hp;
-    c.in_bs = (long)M * N * hp; c.out_bs = (long)N * N * hp;
-    c.bps = 6;
-    {
-      ProfScope p(s, AZB_PROF_FWD_AX0);
-      if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 6L * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
-    }
-  } else {
-    // K1: inverse along axis 0; state [c][i][k] -> X[c][i'][hp]
-    c.in = u_in; c.out = s->X; c.nq = 1;
-    c.in_qs = 0; c.out_qs = 0;
-    c.in_rs = nh; c.out_rs = hp;
-    c.in_bs = (long)N * nh; c.out_bs = (long)M * hp;
-    c.bps = 2;
-    {
-      ProfScope p(s, AZB_PROF_INV_AX0);
-      if ((rc = launch_col<double, T, T, +1, COL_PAD_IN>(M, c, 2L * S, st, s->tsdiv[AZB_PROF_INV_AX0], s->plan[AZB_PROF_INV_AX0]))) return rc;
-    }
-    // K2: last axis; X[c][i'][hp] -> Z[m][i'][hp]
-    r.in = s->X; r.out = s->Z; r.nlines = M;
-    r.in_ss = 2L * M * hp; r.out_ss = 3L * M * hp;
-    {
-      ProfScope p(s, AZB_PROF_ROW);
-      if ((rc = launch_row<T, 2>(M, r, S, st, s->pdiv))) return rc;
-    }
-    // K3: forward along axis 0; Z[m][i'][hp] -> Y[m][i][hp]
-    c.in = s->Z; c.out = s->Y; c.nq = 1;
-    c.in_qs = 0; c.out_qs = 0;
-    c.in_rs = hp; c.out_rs = hp;
-    c.in_bs = (long)M * hp; c.out_bs = (long)N * hp;
-    c.bps = 3;
-    {
-      ProfScope p(s, AZB_PROF_FWD_AX0);
-      if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 3L * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
-    }
+  r.norm = 1.0 / (std::pow(std::sqrt((double)N), 3) * std::pow(std::sqrt((double)M), 3));
+  // K1: inverse along axis 0, N -> M rows; state [c][i][j][k] -> X[c][i'][j][hp]
+  c.in = u_in; c.out = s->X; c.nq = N;
+  c.in_qs = nh; c.out_qs = hp;
+  c.in_rs = (long)N * nh; c.out_rs = (long)N * hp;
+  c.in_bs = (long)N * N * nh; c.out_bs = (long)M * N * hp;
+  c.bps = 3;
+  {
+    ProfScope p(s, AZB_PROF_INV_AX0);
+    if ((rc = launch_col<double, T, T, +1, COL_PAD_IN>(M, c, 3L * S, st, s->tsdiv[AZB_PROF_INV_AX0], s->plan[AZB_PROF_INV_AX0]))) return rc;
   }
-  const double Md = std::pow((double)M, s->dim);
+  // K2: inverse along axis 1; X[c][i'][j][hp] -> Y[c][i'][j'][hp]
+  c.in = s->X; c.out = s->Y; c.nq = 1;
+  c.in_qs = 0; c.out_qs = 0;
+  c.in_rs = hp; c.out_rs = hp;
+  c.in_bs = (long)N * hp; c.out_bs = (long)M * hp;
+  c.bps = 3 * M;
+  {
+    ProfScope p(s, AZB_PROF_INV_AX1);
+    if ((rc = launch_col<T, T, T, +1, COL_PAD_IN>(M, c, 3L * M * S, st, s->tsdiv[AZB_PROF_INV_AX1], s->plan[AZB_PROF_INV_AX1]))) return rc;
+  }
+  // K3: last axis c2r, products, max, r2c; Y[c][line][hp] -> Z[m][line][hp]
+  r.in = s->Y; r.out = s->Z; r.nlines = (long)M * M;
+  r.in_ss = 3L * M * M * hp; r.out_ss = 6L * M * M * hp;
+  {
+    ProfScope p(s, AZB_PROF_ROW);
+    if ((rc = launch_row<T, 3>(M, r, S, st, s->pdiv))) return rc;
+  }
+  // K4: forward along axis 1, M -> N rows; Z[m][i'][j'][hp] -> X[m][i'][j][hp]
+  c.in = s->Z; c.out = s->X; c.nq = 1;
+  c.in_qs = 0; c.out_qs = 0;
+  c.in_rs = hp; c.out_rs = hp;
+  c.in_bs = (long)M * hp; c.out_bs = (long)N * hp;
+  c.bps = 6 * M;
+  {
+    ProfScope p(s, AZB_PROF_FWD_AX1);
+    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 6L * M * S, st, s->tsdiv[AZB_PROF_FWD_AX1], s->plan[AZB_PROF_FWD_AX1]))) return rc;
+  }
+  // K5: forward along axis 0; X[m][i'][j][hp] -> Y[m][i][j][hp] (B_hat on the N-grid)
+  c.in = s->X; c.out = s->Y; c.nq = N;
+  c.in_qs = hp; c.out_qs = hp;
+  c.in_rs = (long)N * hp; c.out_rs = (long)N * hp;
+  c.in_bs = (long)M * N * hp; c.out_bs = (long)N * N * hp;
+  c.bps = 6;
+  {
+    ProfScope p(s, AZB_PROF_FWD_AX0);
+    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 6L * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
+  }
+  const double Md = std::pow((double)M, 3);
   KArgs k{};
-  // 2D: the max|u| reduction runs inside the k-space kernel (a launch less per RHS
-  // where launches are short); 3D keeps it in its own one-workgroup kernel rather
-  // than have each of a million waves re-read the bins at stage 1
-  k.fold = s->dim == 2 ? 1 : 0;
-  k.slot = slot;
-  k.Md = Md;
-  k.C = C;
-  k.Nd = (double)N;
-  if (!k.fold)
-    hipLaunchKernelGGL(finalize_umax, dim3((unsigned)S), dim3(64), 0, st, s->st, slot, kmode == K_RK1 ? 1 : 0,
-                       Md, C, (double)N);
+  hipLaunchKernelGGL(finalize_umax, dim3((unsigned)S), dim3(64), 0, st, s->st, slot, kmode == K_RK1 ? 1 : 0, Md, C,
+                     (double)N);
   k.bh = s->Y;
   k.u_in = u_in;
   k.u0 = u0;
@@ -415,7 +378,7 @@ int enqueue_rhs_T(azb_solver* s, const double2* u_in, const double2* u0, double2
   k.n = N;
   k.nh = nh;
   k.nhp = (int)hp;
-  k.bstride = s->dim == 3 ? (long)N * N * hp : (long)N * hp;
+  k.bstride = (long)N * N * hp;
   k.eps = s->visc.eps;
   k.s2 = 2 * s->visc.s;
   k.k0 = s->visc.k0;
@@ -424,24 +387,181 @@ int enqueue_rhs_T(azb_solver* s, const double2* u_in, const double2* u0, double2
   const unsigned blocks = (unsigned)((s->nmodes + 255) / 256);
   {
     ProfScope p(s, AZB_PROF_KSPACE);
-    launch_kspace((int)sizeof(T), s->dim, k, blocks, (unsigned)S, st);
+    launch_kspace((int)sizeof(T), 3, k, blocks, (unsigned)S, st);
+  }
+  HIPCHK(hipGetLastError());
+  return AZB_OK;
+}
+
+// How one RHS evaluation sits in a sequence of them (2D column stage).
+struct RhsSeq {
+  bool lead = true;      // the inverse passes over u_in are still to be run
+  bool follow = false;   // another evaluation, of `out`, is queued next on this solver
+  bool begin = false;    // first stage of a loop step whose start no kernel has recorded yet
+  bool advance = false;  // last stage of a step of the device-driven loop
+};
+
+// Whether a 2D solver's evaluations run the column stage kernel: where its shape rule says
+// so, with the default radix plans (the kernel's own).
+bool stage_fused(const azb_solver* s) {
+  return s->stage.width > 0 && s->plan[AZB_PROF_INV_AX0] == 0 && s->plan[AZB_PROF_FWD_AX0] == 0;
+}
+
+// 2D row kernel over X -> Z, both [component][line][k] with line stride ls, or in column
+// blocks of bw modes (ls = bw)
+template <typename T>
+int enqueue_row_2d(azb_solver* s, int slot, bool begin, long ls, int bw, long comp) {
+  const int N = s->N, M = s->M;
+  RowArgs r{};
+  r.tw = s->tw;
+  r.st = s->st;
+  r.slot = slot;
+  r.begin = begin ? 1 : 0;
+  r.ls = ls;
+  r.bw = bw;
+  r.norm = 1.0 / (std::pow(std::sqrt((double)N), 2) * std::pow(std::sqrt((double)M), 2));
+  r.in = s->X; r.out = s->Z; r.nlines = M;
+  r.in_ss = 2 * comp; r.out_ss = 3 * comp;
+  ProfScope p(s, AZB_PROF_ROW);
+  return launch_row<T, 2>(M, r, s->S, s->stream);
+}
+
+// 2D, column stage: [inverse of u_in] -> row kernel -> column stage (forward, k-space
+// update, inverse of the new stage value for the next evaluation)
+template <typename T>
+int enqueue_rhs_2d(azb_solver* s, const double2* u_in, const double2* u0, double2* out, int kmode,
+                   int slot, double C, const RhsSeq& seq) {
+  const int N = s->N, M = s->M, nh = s->nh, bw = s->stage.width;
+  StageArgs g{};
+  g.s2 = s->Z;
+  g.u_in = u_in;
+  g.u0 = u0;
+  g.out = out;
+  g.modes = s->modes;
+  g.nh = nh;
+  g.Md = std::pow((double)M, 2);
+  g.C = C;
+  g.Nd = (double)N;
+  g.tw_f = g.tw_i = s->tw;
+  if (sizeof(T) == 4 && M == 768) {
+    g.tw_f = (const cx<T>*)s->tw + col_ptab_offset(0, -1);
+    g.tw_i = (const cx<T>*)s->tw + col_ptab_offset(0, +1);
+  }
+  g.st = s->st;
+  g.slot = slot;
+  g.clear = -1;
+  const std::string not_built = "column length " + std::to_string(M) + " not built";
+  if (seq.lead) {
+    g.mode = K_LEAD;
+    g.x = s->X;
+    ProfScope p(s, AZB_PROF_INV_AX0);
+    if (launch_stage((int)sizeof(T), M, g, s->S, s->stage, s->stream)) return fail(AZB_ERR_UNSUPPORTED, not_built);
+  }
+  int rc;
+  if ((rc = enqueue_row_2d<T>(s, slot, seq.begin, bw, bw, (nh + bw - 1) / bw * (long)bw * M))) return rc;
+  g.mode = kmode;
+  // the solver's own stage buffers are in column blocks too
+  g.in_blocked = kmode == K_RK2 || kmode == K_RK3;
+  g.out_blocked = kmode == K_RK1 || kmode == K_RK2;
+  g.x = seq.follow ? s->X : nullptr;
+  // the previous stage's max|u| bins: read by its own column stage, next filled by a
+  // later stage's row kernel
+  if (kmode != K_DUDT) g.clear = (slot + 2) % 3;
+  g.advance = seq.advance ? 1 : 0;
+  {
+    ProfScope p(s, AZB_PROF_FWD_AX0);
+    if (launch_stage((int)sizeof(T), M, g, s->S, s->stage, s->stream)) return fail(AZB_ERR_UNSUPPORTED, not_built);
+  }
+  HIPCHK(hipGetLastError());
+  return AZB_OK;
+}
+
+// 2D, separate passes: inverse axis 0 -> row kernel -> forward axis 0 -> k-space
+template <typename T>
+int enqueue_rhs_2d_passes(azb_solver* s, const double2* u_in, const double2* u0, double2* out, int kmode,
+                          int slot, double C) {
+  const int N = s->N, M = s->M, nh = s->nh;
+  const long S = s->S, hp = s->nhp;
+  hipStream_t st = s->stream;
+  int rc;
+  ColArgs c{};
+  c.nsmall = N;
+  c.tw = s->tw;
+  c.st = s->st;
+  c.nk = nh;
+  c.nq = 1;
+  // state [c][i][k] -> X[c][i'][hp]
+  c.in = u_in; c.out = s->X;
+  c.in_rs = nh; c.out_rs = hp;
+  c.in_bs = (long)N * nh; c.out_bs = (long)M * hp;
+  c.bps = 2;
+  {
+    ProfScope p(s, AZB_PROF_INV_AX0);
+    if ((rc = launch_col<double, T, T, +1, COL_PAD_IN>(M, c, 2L * S, st, s->tsdiv[AZB_PROF_INV_AX0], s->plan[AZB_PROF_INV_AX0]))) return rc;
+  }
+  if ((rc = enqueue_row_2d<T>(s, slot, false, hp, 0, M * hp))) return rc;
+  // Z[m][i'][hp] -> Y[m][i][hp]
+  c.in = s->Z; c.out = s->Y;
+  c.in_rs = hp; c.out_rs = hp;
+  c.in_bs = (long)M * hp; c.out_bs = (long)N * hp;
+  c.bps = 3;
+  {
+    ProfScope p(s, AZB_PROF_FWD_AX0);
+    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 3L * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
+  }
+  KArgs k{};
+  // the max|u| reduction runs inside the k-space kernel (a launch less per RHS where
+  // launches are short)
+  k.fold = 1;
+  k.slot = slot;
+  k.Md = std::pow((double)M, 2);
+  k.C = C;
+  k.Nd = (double)N;
+  k.bh = s->Y;
+  k.u_in = u_in;
+  k.u0 = u0;
+  k.out = out;
+  k.nmodes = s->nmodes;
+  k.n = N;
+  k.nh = nh;
+  k.nhp = (int)hp;
+  k.bstride = (long)N * hp;
+  k.eps = s->visc.eps;
+  k.s2 = 2 * s->visc.s;
+  k.k0 = s->visc.k0;
+  k.mode = kmode;
+  k.st = s->st;
+  {
+    ProfScope p(s, AZB_PROF_KSPACE);
+    launch_kspace((int)sizeof(T), 2, k, (unsigned)((s->nmodes + 255) / 256), (unsigned)S, st);
   }
   HIPCHK(hipGetLastError());
   return AZB_OK;
 }
 
 int enqueue_rhs(azb_solver* s, const double2* u_in, const double2* u0, double2* out, int kmode,
-                int slot, double C) {
-  if (s->prec == AZB_FP64) return enqueue_rhs_T<double>(s, u_in, u0, out, kmode, slot, C);
-  return enqueue_rhs_T<float>(s, u_in, u0, out, kmode, slot, C);
+                int slot, double C, const RhsSeq& seq = {}) {
+  if (stage_fused(s))
+    return s->prec == AZB_FP64 ? enqueue_rhs_2d<double>(s, u_in, u0, out, kmode, slot, C, seq)
+                               : enqueue_rhs_2d<float>(s, u_in, u0, out, kmode, slot, C, seq);
+  if (s->dim == 2)
+    return s->prec == AZB_FP64 ? enqueue_rhs_2d_passes<double>(s, u_in, u0, out, kmode, slot, C)
+                               : enqueue_rhs_2d_passes<float>(s, u_in, u0, out, kmode, slot, C);
+  return s->prec == AZB_FP64 ? enqueue_rhs_3d<double>(s, u_in, u0, out, kmode, slot, C)
+                             : enqueue_rhs_3d<float>(s, u_in, u0, out, kmode, slot, C);
 }
 
-// the three stages of SSP_RK3::integrate (ssp_rk3.hpp:54-62), stage updates fused
-int enqueue_rk3_stages(azb_solver* s, double2* u, double C) {
+// the three stages of SSP_RK3::integrate (ssp_rk3.hpp:54-62), stage updates fused.  With
+// the 2D column stage the inverse passes of every stage but the first of a sequence run at the end of the
+// stage before it: `lead` false when the previous step did this step's, `follow` when
+// another step of the same state comes next; `loop`: a step of the device-driven loop.
+int enqueue_rk3_stages(azb_solver* s, double2* u, double C, bool lead = true, bool follow = false,
+                       bool loop = false) {
   int rc;
-  if ((rc = enqueue_rhs(s, u, nullptr, s->u1, K_RK1, 0, C))) return rc;   // u1 = u + dt L(u)
-  if ((rc = enqueue_rhs(s, s->u1, u, s->u2, K_RK2, 1, C))) return rc;     // u2 = 3/4 u + 1/4 (u1 + dt L(u1))
-  if ((rc = enqueue_rhs(s, s->u2, u, u, K_RK3, 2, C))) return rc;         // u = 2/3 (u2 + dt L(u2)) + 1/3 u
+  const RhsSeq q1{lead, true, loop && !lead, false}, q2{false, true, false, false}, q3{false, follow, false, loop};
+  if ((rc = enqueue_rhs(s, u, nullptr, s->u1, K_RK1, 0, C, q1))) return rc;   // u1 = u + dt L(u)
+  if ((rc = enqueue_rhs(s, s->u1, u, s->u2, K_RK2, 1, C, q2))) return rc;     // u2 = 3/4 u + 1/4 (u1 + dt L(u1))
+  if ((rc = enqueue_rhs(s, s->u2, u, u, K_RK3, 2, C, q3))) return rc;         // u = 2/3 (u2 + dt L(u2)) + 1/3 u
   return AZB_OK;
 }
 
@@ -463,6 +583,7 @@ int check_solver_args(int dim, int N, int M, int n_vars, int precision, int nsam
 // bytes of the intermediates X, Y, Z and of one RK stage buffer for S samples
 struct Layout {
   size_t xs, ys, zs, us;
+  size_t ms;  // 2D mode table, shared by the samples
 };
 
 // fill a solver's grid fields (arguments already checked); no allocation
@@ -495,8 +616,12 @@ Layout setup_solver(azb_solver* s, int dim, int N, int precision, azb_sv_params 
     l.xs = S * cs * 2 * (size_t)M * hp;
     l.ys = S * cs * 3 * (size_t)N * hp;
     l.zs = S * cs * 3 * (size_t)M * hp;
+    s->stage = stage_shape((int)s->tsize, M, nsamples);
+    if (s->stage.width) l.ms = sizeof(double2) * s->nmodes;
   }
   l.us = S * sizeof(double2) * (size_t)dim * s->nmodes;
+  if (s->stage.width)  // in column blocks
+    l.us = S * sizeof(double2) * 2 * (size_t)N * ((nh + s->stage.width - 1) / s->stage.width * s->stage.width);
   return l;
 }
 
@@ -577,17 +702,17 @@ int azb_create_batch(int dim, int N, int M, int n_vars, int precision, azb_sv_pa
   if (rc) return rc;
   azb_solver* s = new azb_solver();
   const Layout lay = setup_solver(s, dim, N, precision, visc, nsamples);
-  const size_t xs = lay.xs, ys = lay.ys, zs = lay.zs, us = lay.us, S = nsamples;
+  const size_t xs = lay.xs, ys = lay.ys, zs = lay.zs, us = lay.us, ms = lay.ms, S = nsamples;
   auto cleanup = [&](int code, const std::string& m) {
     azb_destroy(s);
     return fail(code, m);
   };
   if (hipMalloc(&s->X, xs) != hipSuccess || hipMalloc(&s->Y, ys) != hipSuccess ||
-      hipMalloc(&s->Z, zs) != hipSuccess || hipMalloc((void**)&s->u1, us) != hipSuccess ||
+      hipMalloc(&s->Z, zs) != hipSuccess || (ms && hipMalloc((void**)&s->modes, ms) != hipSuccess) || hipMalloc((void**)&s->u1, us) != hipSuccess ||
       hipMalloc((void**)&s->u2, us) != hipSuccess ||
       hipMalloc((void**)&s->st, S * sizeof(DevState)) != hipSuccess)
     return cleanup(AZB_ERR_ALLOC, "device allocation of the solver workspace failed");
-  s->bytes = xs + ys + zs + 2 * us + S * sizeof(DevState);
+  s->bytes = xs + ys + zs + 2 * us + ms + S * sizeof(DevState);
   rc = precision == AZB_FP64 ? make_twiddles<double>(s->M, &s->tw) : make_twiddles<float>(s->M, &s->tw);
   if (rc) {
     std::string m = g_err;
@@ -597,6 +722,10 @@ int azb_create_batch(int dim, int N, int M, int n_vars, int precision, azb_sv_pa
   std::vector<DevState> h(S);
   if (hipMemcpy(s->st, h.data(), S * sizeof(DevState), hipMemcpyHostToDevice) != hipSuccess)
     return cleanup(AZB_ERR_HIP, "hipMemcpy of the device state failed");
+  if (s->modes) {
+    launch_stage_modes(s->modes, N, visc.eps, 2 * visc.s, visc.k0, s->stream);
+    if (hipGetLastError() != hipSuccess) return cleanup(AZB_ERR_HIP, "launch of the mode table kernel failed");
+  }
   *out = s;
   return AZB_OK;
 }
@@ -611,15 +740,17 @@ int azb_num_samples(const azb_solver* s) { return s ? s->S : 0; }
 size_t azb_bytes_estimate(int dim, int N, int precision, int nsamples) {
   const size_t cs = precision == AZB_FP64 ? 16 : 8;
   const size_t M = 3 * (size_t)N / 2, nh = N / 2 + 1, hp = (nh + 15) / 16 * 16, S = nsamples;
-  size_t ws, us;
+  size_t ws, us, ms = 0;
   if (dim == 3) {
     ws = cs * (6 * M * N * hp + std::max(3 * M * M * hp, 6 * (size_t)N * N * hp) + 6 * M * M * hp);
     us = sizeof(double2) * 3 * (size_t)N * N * nh;
   } else {
     ws = cs * (2 * M * hp + 3 * (size_t)N * hp + 3 * M * hp);
-    us = sizeof(double2) * 2 * (size_t)N * nh;
+    const size_t w = stage_shape(precision == AZB_FP64 ? 8 : 4, (int)M, nsamples).width;
+    us = sizeof(double2) * 2 * (size_t)N * (w ? (nh + w - 1) / w * w : nh);
+    ms = w ? sizeof(double2) * (size_t)N * nh : 0;
   }
-  return S * (ws + 2 * us + sizeof(DevState));
+  return S * (ws + 2 * us + sizeof(DevState)) + ms;
 }
 
 int azb_destroy(azb_solver* s) {
@@ -628,6 +759,7 @@ int azb_destroy(azb_solver* s) {
   (void)hipFree(s->X);
   (void)hipFree(s->Y);
   (void)hipFree(s->Z);
+  (void)hipFree(s->modes);
   (void)hipFree(s->u1);
   (void)hipFree(s->u2);
   (void)hipFree(s->st);
@@ -660,7 +792,8 @@ int azb_dudt_noalloc(int dim, int N, int precision, azb_sv_params visc, const vo
   if (rc) return rc;
   azb_solver s;  // grid fields only: its buffers are carved out of the scratch array below
   const Layout l = setup_solver(&s, dim, N, precision, visc, 1);
-  const size_t xs = round256(l.xs), ys = round256(l.ys), zs = round256(l.zs);
+  // 2D: one sample runs the column stage, which needs its mode table in the place of Y
+  const size_t xs = round256(l.xs), ys = round256(dim == 2 ? l.ms : l.ys), zs = round256(l.zs);
   const size_t need = xs + ys + zs + round256(sizeof(DevState));
   if (need > kScratchBytes - kScratchTwBytes)
     return fail(AZB_ERR_UNSUPPORTED, std::to_string(dim) + "D N = " + std::to_string(N) + " needs " +
@@ -676,6 +809,10 @@ int azb_dudt_noalloc(int dim, int N, int precision, azb_sv_params visc, const vo
   s.Z = w + xs + ys;
   s.st = (DevState*)(w + xs + ys + zs);
   s.stream = (hipStream_t)stream;
+  if (dim == 2) {
+    s.modes = (double2*)s.Y;
+    launch_stage_modes(s.modes, N, visc.eps, 2 * visc.s, visc.k0, s.stream);
+  }
   // clears the max|u| bins the previous call on this GPU left in the array
   hipLaunchKernelGGL(step_prologue_fixed, dim3(1), dim3(256), 0, s.stream, s.st, 0.0);
   return enqueue_rhs(&s, (const double2*)u_hat, nullptr, (double2*)dudt_hat, K_DUDT, 3, 0.0);
@@ -744,11 +881,15 @@ int azb_loop_begin_sample(azb_solver* s, int sample, double t_end, double C, dou
 
 int azb_enqueue_steps(azb_solver* s, void* u_hat, int nsteps) {
   if (!s || !u_hat) return fail(AZB_ERR_ARG, "NULL argument");
+  // with the 2D column stage the steps of one call run without control kernels between
+  // them: the last stage advances the time, the next step's row kernel starts it
+  const bool fused = stage_fused(s);
   for (int i = 0; i < nsteps; ++i) {
-    hipLaunchKernelGGL(step_prologue_loop, dim3(s->S), dim3(256), 0, s->stream, s->st);
-    int rc = enqueue_rk3_stages(s, (double2*)u_hat, s->loop_C);
+    const bool lead = !fused || i == 0;
+    if (lead) hipLaunchKernelGGL(step_prologue_loop, dim3(s->S), dim3(256), 0, s->stream, s->st);
+    int rc = enqueue_rk3_stages(s, (double2*)u_hat, s->loop_C, lead, i + 1 < nsteps, fused);
     if (rc) return rc;
-    hipLaunchKernelGGL(step_epilogue_loop, dim3(s->S), dim3(64), 0, s->stream, s->st);
+    if (!fused) hipLaunchKernelGGL(step_epilogue_loop, dim3(s->S), dim3(64), 0, s->stream, s->st);
   }
   HIPCHK(hipGetLastError());
   return AZB_OK;
@@ -1046,6 +1187,10 @@ int azb_autotune_plans(azb_solver* s, const void* u_hat, int reps) {
   if (reps < 1) reps = 3;
   const int n = col_plan_count(s->M);
   if (n == 1) return AZB_OK;
+  if (s->stage.width) {  // the column stage is built for plan 0 and chosen where it beats the separate passes
+    const int zero[AZB_PROF_FAMILIES] = {};
+    return azb_set_plans(s, zero);
+  }
   const bool prof_was = s->prof;
   int keep[AZB_PROF_FAMILIES], pick[AZB_PROF_FAMILIES];
   double best[AZB_PROF_FAMILIES];
