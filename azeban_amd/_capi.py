@@ -75,6 +75,9 @@ SIGNATURES = {
     "azb_fft_work_init": (_i, [_vp, _i, _i]),
     "azb_fft_r2c_ws": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "azb_fft_c2r_ws": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp]),
+    "azb_fft_shared_work": (_i, [_i, _i, C.POINTER(_vp)]),
+    "azb_fft_c2r_from": (_i, [_i, _i, _i, _i, _d, _vp, _vp, _vp, _vp, _vp]),
+    "azb_initialize": (_i, [_i, _i, _vp, _vp, _vp, _vp]),
     "azb_copy_to_padded": (_i, [_i, _i, _i, _vp, _vp, _vp]),
     "azb_copy_from_padded": (_i, [_i, _i, _i, _vp, _vp, _vp]),
     "azb_scale": (_i, [_d, _vp, _l, _vp]),

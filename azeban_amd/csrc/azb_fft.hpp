@@ -47,12 +47,17 @@ __device__ __forceinline__ cx<T> gload(const void* base, unsigned idx) {
 // non-temporal stores the column passes measured 5-9 % faster.  Loads stay cached
 // (neighbouring tiles share the lines that straddle tile boundaries; non-temporal
 // loads measured 7-25 % slower).
-template <typename T>
+// STREAM = false: cached stores, where rows are not line-aligned and the neighbouring
+// tile completes the lines.
+template <typename T, bool STREAM = true>
 __device__ __forceinline__ void gstore(void* base, unsigned idx, T x, T y) {
   vec2_t<T> v;
   v.x = x;
   v.y = y;
-  __builtin_nontemporal_store(v, &((gvec2<T>*)base)[idx]);
+  if (STREAM)
+    __builtin_nontemporal_store(v, &((gvec2<T>*)base)[idx]);
+  else
+    ((gvec2<T>*)base)[idx] = v;
 }
 
 template <typename T>
@@ -316,148 +321,6 @@ constexpr long plan_prod() { return R0; }
 template <int R0, int R1, int... Rs>
 constexpr long plan_prod() { return (long)R0 * plan_prod<R1, Rs...>(); }
 
-// LDS words needed by the exchange (SPLIT: one T per element, else two)
-template <typename T, int L, int TS, bool SPLIT>
-struct ExchangeSize {
-  static constexpr int words = TS * L * (SPLIT ? 1 : 2);
-};
-
-template <typename T, int L, int TS, int NT, int DIR, bool SPLIT>
-struct BlockFFT {
-  static constexpr int E = TS * L / NT;
-  static_assert(TS * L % NT == 0, "TS*L must be a multiple of NT");
-
-  // twiddle W_L^{e} with direction applied; the table pointer is in the global
-  // address space: global (not flat) loads
-  // with a scalar base and a 32-bit offset, and no flat-load entries in the LDS
-  // wait counter
-  using twptr = const __attribute__((address_space(1))) cx<T>*;
-
-  __device__ __forceinline__ static cx<T> twiddle(twptr tw, unsigned e) {
-    cx<T> w;
-    w.x = tw[e].x;
-    w.y = DIR > 0 ? -tw[e].y : tw[e].y;
-    return w;
-  }
-
-  template <int Ns, int R>
-  __device__ __forceinline__ static void butterflies(cx<T>* v, int t, const cx<T>* __restrict__ tw) {
-    static_assert(E % R == 0, "radix must divide E");
-#pragma unroll
-    for (int b = 0; b < E / R; ++b) {
-      cx<T>* w = v + b * R;
-      if (Ns > 1) {
-        const unsigned g = (unsigned)t + NT * b;
-        const unsigned j = g / TS;
-        const unsigned k = j % Ns;
-        constexpr unsigned step = L / (Ns * R);
-#pragma unroll
-        for (int r = 1; r < R; ++r) w[r] = cmul(w[r], twiddle((twptr)tw, r * k * step));
-      }
-      DFT<R, DIR, T>::run(w);
-    }
-  }
-
-  // write pass (Ns,R) outputs into LDS in [pos][s] order, then read the next pass's inputs
-  template <int Ns, int R, int Rn>
-  __device__ __forceinline__ static void exchange(cx<T>* v, int t, T* lds, bool active) {
-    constexpr int comps = SPLIT ? 2 : 1;
-#pragma unroll
-    for (int c = 0; c < comps; ++c) {
-      __syncthreads();
-      if (active) {
-#pragma unroll
-        for (int b = 0; b < E / R; ++b) {
-          const unsigned g = (unsigned)t + NT * b;
-          const unsigned s = g % TS;
-          const unsigned j = g / TS;
-          const unsigned k = j % Ns;
-          const unsigned base = (j - k) * R + k;
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const unsigned idx = (base + r * Ns) * TS + s;
-            if (SPLIT) {
-              lds[idx] = c == 0 ? v[b * R + r].x : v[b * R + r].y;
-            } else {
-              lds[2 * idx] = v[b * R + r].x;
-              lds[2 * idx + 1] = v[b * R + r].y;
-            }
-          }
-        }
-      }
-      __syncthreads();
-      if (active) {
-#pragma unroll
-        for (int b = 0; b < E / Rn; ++b) {
-          const unsigned g = (unsigned)t + NT * b;
-          const unsigned s = g % TS;
-          const unsigned j = g / TS;
-#pragma unroll
-          for (int r = 0; r < Rn; ++r) {
-            const unsigned idx = (j + r * (L / Rn)) * TS + s;
-            if (SPLIT) {
-              if (c == 0)
-                v[b * Rn + r].x = lds[idx];
-              else
-                v[b * Rn + r].y = lds[idx];
-            } else {
-              v[b * Rn + r].x = lds[2 * idx];
-              v[b * Rn + r].y = lds[2 * idx + 1];
-            }
-          }
-        }
-      }
-    }
-  }
-
-  template <int Ns, int R>
-  __device__ __forceinline__ static void passes(cx<T>* v, int t, T* lds, const cx<T>* tw,
-                                                bool active, Plan<R>) {
-    if (active) butterflies<Ns, R>(v, t, tw);
-  }
-  template <int Ns, int R, int Rn, int... Rs>
-  __device__ __forceinline__ static void passes(cx<T>* v, int t, T* lds, const cx<T>* tw,
-                                                bool active, Plan<R, Rn, Rs...>) {
-    if (active) butterflies<Ns, R>(v, t, tw);
-    exchange<Ns, R, Rn>(v, t, lds, active);
-    passes<Ns * R, Rn, Rs...>(v, t, lds, tw, active, Plan<Rn, Rs...>{});
-  }
-
-  // Run the whole transform.  All threads of the workgroup must call this (it holds
-  // barriers); threads with active == false only take part in the barriers.
-  template <int... Rs>
-  __device__ __forceinline__ static void run(cx<T>* v, int t, T* lds, const cx<T>* tw, bool active,
-                                             Plan<Rs...> p) {
-    static_assert(plan_prod<Rs...>() == L, "plan must multiply to L");
-    passes<1, Rs...>(v, t, lds, tw, active, p);
-  }
-
-  // first-pass load: ld(s, pos) -> cx<T>
-  template <int R0, class Ld>
-  __device__ __forceinline__ static void load(cx<T>* v, int t, Ld ld) {
-#pragma unroll
-    for (int b = 0; b < E / R0; ++b) {
-      const unsigned g = (unsigned)t + NT * b;
-      const unsigned s = g % TS;
-      const unsigned j = g / TS;
-#pragma unroll
-      for (int r = 0; r < R0; ++r) v[b * R0 + r] = ld(s, j + r * (L / R0));
-    }
-  }
-  // last-pass store: st(s, pos, value)
-  template <int RL, class St>
-  __device__ __forceinline__ static void store(const cx<T>* v, int t, St st) {
-#pragma unroll
-    for (int b = 0; b < E / RL; ++b) {
-      const unsigned g = (unsigned)t + NT * b;
-      const unsigned s = g % TS;
-      const unsigned j = g / TS;
-#pragma unroll
-      for (int r = 0; r < RL; ++r) st(s, j + r * (L / RL), v[b * RL + r]);
-    }
-  }
-};
-
 }  // namespace azb
 
 namespace azb {
@@ -587,8 +450,9 @@ struct LayElems<void, D> {
 
 // Twiddles and butterfly j of one Stockham pass (accumulated size Ns, radix R) on the
 // R values w: w_r *= W_{Ns R}^{r (j mod Ns)}, then DFT_R.  PTAB: tw is the pass's
-// per-pass table (see BlockFFT2), else the W_L^e table.
-template <typename T, int L, int DIR, int Ns, int R, bool PTAB>
+// per-pass table (see BlockFFT2), else the W_L^e table, read for every power or (CHAIN) once
+// per butterfly.
+template <typename T, int L, int DIR, int Ns, int R, bool PTAB, bool CHAIN = sizeof(T) == 8>
 __device__ __forceinline__ void butterfly(cx<T>* w, const __attribute__((address_space(1))) cx<T>* tw, unsigned j) {
   if constexpr (Ns > 1) {
     auto twiddle = [&](unsigned e) -> cx<T> {
@@ -612,8 +476,8 @@ __device__ __forceinline__ void butterfly(cx<T>* w, const __attribute__((address
         w[2 * q + 1] = cmul(w[2 * q + 1], mk(T(two.x), T(two.y)));
         if (2 * q + 2 < R) w[2 * q + 2] = cmul(w[2 * q + 2], mk(T(two.z), T(two.w)));
       }
-    } else if constexpr (sizeof(T) == 8) {
-      // FP64: one table load per butterfly, the other powers by repeated
+    } else if constexpr (CHAIN) {
+      // FP64 kernels bound by issue: one table load per butterfly, the other powers by repeated
       // multiplication (w^(r+1) = w^r w, below 22 ulp at R = 24).  Each saved
       // load is a full vector-memory instruction through the texture path; the
       // chain costs four FMA-class operations and keeps two powers live.
@@ -628,7 +492,7 @@ __device__ __forceinline__ void butterfly(cx<T>* w, const __attribute__((address
         w[r] = cmul_fixed(w[r], wr);
       }
     } else {
-      // FP32 loads every power: a chain's error would rival the transform's own
+      // every power from the table: in FP32 a chain's error would rival the transform's own
 #pragma unroll
       for (int r = 1; r < R; ++r) w[r] = cmul(w[r], twiddle(r * k * step));
     }
@@ -648,7 +512,7 @@ __device__ __forceinline__ void butterfly(cx<T>* w, const __attribute__((address
 // r = 1 .. R-1 at row[r-1]) instead of the W_L^e table: one base address per
 // butterfly, constant offsets, 16-byte loads of two FP32 entries.
 template <typename T, int L, int TS, int NT, int DIR, bool SPLIT, int G, int MAPF, int MAPL, bool SWZ = false,
-          int SOFF = 1, unsigned MIDW = 0, int PADE = 0, unsigned MIDH = 0, class LSEL = void, bool PTAB = false>
+          int SOFF = 1, unsigned MIDW = 0, int PADE = 0, unsigned MIDH = 0, class LSEL = void, bool PTAB = false, bool CHAIN = sizeof(T) == 8>
 struct BlockFFT2 {
   static constexpr int E = TS * L / NT;
   static_assert(TS * L % NT == 0, "TS*L must be a multiple of NT");
@@ -709,7 +573,7 @@ struct BlockFFT2 {
     for (int b = 0; b < E / R; ++b) {
       unsigned s = 0, j = 0;
       if (Ns > 1) bmap<MAP, TS, NT, L, R, G>(t, b, s, j);
-      butterfly<T, L, DIR, Ns, R, PTAB>(v + b * R, tw, j);
+      butterfly<T, L, DIR, Ns, R, PTAB, CHAIN>(v + b * R, tw, j);
     }
   }
 

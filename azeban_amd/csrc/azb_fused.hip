@@ -101,19 +101,27 @@ int launch_row_fused(int tbytes, int dim, int L, const RowArgs& a, long nsamples
                   : launch_row_T<float, 2>(L, a, nsamples, st, pdiv);
 }
 
-void launch_kspace(int tbytes, int dim, const KArgs& k, unsigned blocks, unsigned samples, hipStream_t st) {
-  const dim3 grid(blocks, samples), block(256);
-  if (tbytes == 8) {
-    if (dim == 3)
-      hipLaunchKernelGGL((kspace_kernel<double, 3>), grid, block, 0, st, k);
-    else
-      hipLaunchKernelGGL((kspace_kernel<double, 2>), grid, block, 0, st, k);
-  } else {
-    if (dim == 3)
-      hipLaunchKernelGGL((kspace_kernel<float, 3>), grid, block, 0, st, k);
-    else
-      hipLaunchKernelGGL((kspace_kernel<float, 2>), grid, block, 0, st, k);
+namespace {
+
+template <typename T, int DIM>
+void launch_kspace_T(const KArgs& k, dim3 grid, hipStream_t st) {
+  const dim3 block(256);
+  switch (k.mode) {
+    case K_RK1: hipLaunchKernelGGL((kspace_kernel<T, DIM, K_RK1>), grid, block, 0, st, k); break;
+    case K_RK2: hipLaunchKernelGGL((kspace_kernel<T, DIM, K_RK2>), grid, block, 0, st, k); break;
+    case K_RK3: hipLaunchKernelGGL((kspace_kernel<T, DIM, K_RK3>), grid, block, 0, st, k); break;
+    default: hipLaunchKernelGGL((kspace_kernel<T, DIM, K_DUDT>), grid, block, 0, st, k); break;
   }
+}
+
+}  // namespace
+
+void launch_kspace(int tbytes, int dim, const KArgs& k, unsigned blocks, unsigned samples, hipStream_t st) {
+  const dim3 grid(blocks, samples);
+  if (tbytes == 8)
+    dim == 3 ? launch_kspace_T<double, 3>(k, grid, st) : launch_kspace_T<double, 2>(k, grid, st);
+  else
+    dim == 3 ? launch_kspace_T<float, 3>(k, grid, st) : launch_kspace_T<float, 2>(k, grid, st);
 }
 
 namespace {

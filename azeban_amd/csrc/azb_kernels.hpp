@@ -103,6 +103,7 @@ struct ColArgs {
   int bps;              // batches per sample (samples are stacked batch-major)
   const void* tw;       // twiddles for L
   const DevState* st;   // one per sample
+  double scale;         // COL_FULL: factor of the input
 };
 
 // columns per workgroup: 128-byte segments at working precision
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(TS * L / LenPlan<L>::E, (sizeof(T) == 4 ? 4 : (L ==
   using F = BlockFFT2<T, L, TS, NT, DIR, SPLIT, 1, MAP_STD, MAP_STD, false, 1, 0u, 0, 0u, void, PT>;
   constexpr int R0 = first_radix(PP{});
   constexpr int RL = last_radix(PP{});
-  __shared__ T lds[ExchangeSize<T, L, TS, SPLIT>::words];
+  __shared__ T lds[F::lds_words];
   const int t = threadIdx.x;
   const unsigned blk = xcd_contiguous(blockIdx.x, gridDim.x);
   const int kt = blk % a.ktiles;
@@ -172,6 +173,7 @@ __global__ __launch_bounds__(TS * L / LenPlan<L>::E, (sizeof(T) == 4 ? 4 : (L ==
     if (valid) {
       const cx<Tin> x = gload<Tin>(in, row * irs + s);
       r = mk(T(x.x), T(x.y));
+      if (MODE == COL_FULL) r = cscale(r, T(a.scale));
     }
     return r;
   });
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(TS * L / LenPlan<L>::E, (sizeof(T) == 4 ? 4 : (L ==
           valid = false;
       }
     }
-    if (valid) gstore<Tout>(out, row * ors + s, Tout(val.x), Tout(val.y));
+    if (valid) gstore<Tout, MODE != COL_FULL>(out, row * ors + s, Tout(val.x), Tout(val.y));
   });
 }
 
@@ -210,10 +212,10 @@ struct RowArgs {
   const void* tw;
   DevState* st;
   int slot;         // umax slot
-  int begin;        // first kernel of a step of the device-driven loop (see row_idle)
+  int begin;        // 2D: first kernel of a step of the device-driven loop (see row_idle)
 };
 
-// Whether this workgroup's sample sits the launch out.  In the first kernel of a loop step
+// 2D: whether this workgroup's sample sits the launch out.  In the first kernel of a loop step
 // every workgroup decides from the sample's time, which no kernel of the previous step
 // still writes, and the sample's first workgroup records the decision and the step's clamp
 // for the kernels that follow (step_prologue_loop's work without its launch).
@@ -261,7 +263,7 @@ struct KArgs {
   int nhp;               // last-axis stride of B_hat (>= nh)
   long bstride;          // component stride of B_hat
   double eps, s2, k0;    // SmoothCutoff1D with s2 = 2s
-  int mode;
+  int mode;              // KMode: the kernel's MODE
   DevState* st;          // one per sample
   // fold = 1 (2D): the max|u| reduction of this RHS runs here instead of in a kernel
   // of its own: u_max = max(bins[slot]) / Md, at stage 1 dt = min(C / (Nd u_max), max_dt)
@@ -366,7 +368,7 @@ __device__ __forceinline__ double stage_value(int mode, double absk2, double L, 
   return (2.0 / 3) * tmp + (1.0 / 3) * w;
 }
 
-template <typename T, int DIM>
+template <typename T, int DIM, int MODE>
 __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
   // grid.y = sample; samples are stacked with strides DIM*nmodes (state) and
   // 3(DIM-1)*bstride (B_hat)
@@ -380,14 +382,14 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
   if (a.fold) {
     const bool first = blockIdx.x == 0;
     double um = 0.0;
-    if (a.mode == K_RK1 || first) {
+    if (MODE == K_RK1 || first) {
       const double v = __longlong_as_double((long long)st->umax_bins[a.slot][threadIdx.x & (kBins - 1)]);
       um = wave_max<double>(v) / a.Md;
     }
-    dt = a.mode == K_RK1 ? fmin(a.C / (a.Nd * um), st->max_dt) : st->dt;
+    dt = MODE == K_RK1 ? fmin(a.C / (a.Nd * um), st->max_dt) : st->dt;
     if (first && threadIdx.x == 0) {
       st->u_max = um;
-      if (a.mode == K_RK1) st->dt = dt;
+      if (MODE == K_RK1) st->dt = dt;
     }
   } else {
     dt = st->dt;
@@ -422,104 +424,11 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
     const long o = (sample * DIM + c) * a.nmodes + idx;
     const cx<double> u = ntload<double>(a.u_in + o);
     cx<double> w = mk(0.0, 0.0);
-    if (a.mode == K_RK2 || a.mode == K_RK3) w = ntload<double>(a.u0 + o);
+    if (MODE == K_RK2 || MODE == K_RK3) w = ntload<double>(a.u0 + o);
     vec2_t<double> rv;
-    rv.x = stage_value(a.mode, g.absk2, Lr[c], nu, u.x, w.x, dt);
-    rv.y = stage_value(a.mode, g.absk2, Li[c], nu, u.y, w.y, dt);
+    rv.x = stage_value(MODE, g.absk2, Lr[c], nu, u.x, w.x, dt);
+    rv.y = stage_value(MODE, g.absk2, Li[c], nu, u.y, w.y, dt);
     __builtin_nontemporal_store(rv, (vec2_t<double>*)(a.out + o));
-  }
-}
-
-}  // namespace azb
-
-namespace azb {
-
-// ---------------------------------------------------------------------------
-// Plain last-axis real transforms (standalone FFT entry points): pairs of real
-// lines share one complex FFT.  c2r drops Im at k = 0 and k = L/2 (FFTW/cuFFT
-// convention); r2c writes the L/2+1 non-negative frequencies.
-// ---------------------------------------------------------------------------
-struct PlainRowArgs {
-  const void* in;
-  void* out;
-  long nlines;
-  const void* tw;
-};
-
-template <typename T, int L, int P, int DIR>
-__global__ __launch_bounds__(2 * P * L / LenPlan<L>::E / 2) void plain_row_kernel(PlainRowArgs a) {
-  // TS = P (one complex FFT per pair of lines)
-  using LP = LenPlan<L>;
-  constexpr int TS = P;
-  constexpr int NT = TS * L / LP::E;
-  constexpr int NH = L / 2 + 1;
-  constexpr bool SPLIT = sizeof(T) == 8;
-  constexpr int R0 = first_radix(typename LP::P{});
-  constexpr int RL = last_radix(typename LP::P{});
-  using F = BlockFFT<T, L, TS, NT, DIR, SPLIT>;
-  __shared__ T X[SPLIT ? TS * L : 2 * TS * L];
-  __shared__ cx<T> stg[DIR > 0 ? 2 * P * NH : 1];
-  const int t = threadIdx.x;
-  const long line0 = (long)blockIdx.x * 2 * P;
-  const cx<T>* tw = (const cx<T>*)a.tw;
-  cx<T> v[LP::E];
-  if (DIR > 0) {
-    const cx<T>* in = (const cx<T>*)a.in;
-    for (int e = t; e < 2 * P * NH; e += NT) {
-      const long line = line0 + e / NH;
-      stg[e] = line < a.nlines ? in[line * NH + e % NH] : mk(T(0), T(0));
-    }
-    __syncthreads();
-    F::template load<R0>(v, t, [&](int s, int pos) -> cx<T> {
-      const cx<T>* xs = stg + (2 * s) * NH;
-      const cx<T>* ys = stg + (2 * s + 1) * NH;
-      if (pos == 0 || pos == L / 2) return mk(xs[pos].x, ys[pos].x);
-      if (pos < L / 2) {
-        const cx<T> X0 = xs[pos], Y0 = ys[pos];
-        return mk(X0.x - Y0.y, X0.y + Y0.x);
-      }
-      const cx<T> X0 = xs[L - pos], Y0 = ys[L - pos];
-      return mk(X0.x + Y0.y, Y0.x - X0.y);
-    });
-    F::run(v, t, X, tw, true, typename LP::P{});
-    T* out = (T*)a.out;
-    F::template store<RL>(v, t, [&](int s, int pos, cx<T> val) {
-      const long la = line0 + 2 * s, lb = la + 1;
-      if (la < a.nlines) out[la * L + pos] = val.x;
-      if (lb < a.nlines) out[lb * L + pos] = val.y;
-    });
-  } else {
-    const T* in = (const T*)a.in;
-    F::template load<R0>(v, t, [&](int s, int pos) -> cx<T> {
-      const long la = line0 + 2 * s, lb = la + 1;
-      const T xa = la < a.nlines ? in[la * L + pos] : T(0);
-      const T xb = lb < a.nlines ? in[lb * L + pos] : T(0);
-      return mk(xa, xb);
-    });
-    F::run(v, t, X, tw, true, typename LP::P{});
-    cx<T>* out = (cx<T>*)a.out;
-    constexpr int items = TS * NH;
-    for (int ph = 0; ph < 2; ++ph) {
-      __syncthreads();
-      F::template store<RL>(v, t, [&](int s, int pos, cx<T> val) {
-        X[s * L + pos] = ph == 0 ? val.x : val.y;
-      });
-      __syncthreads();
-      for (int it = t; it < items; it += NT) {
-        const int k = it % NH, s = it / NH;
-        const T zk = X[s * L + k];
-        const T zm = X[s * L + (k == 0 ? 0 : L - k)];
-        const long la = line0 + 2 * s, lb = la + 1;
-        // stage the first half-result in the output (re-read in phase 1)
-        if (ph == 0) {
-          if (la < a.nlines) out[la * NH + k].x = T(0.5) * (zk + zm);
-          if (lb < a.nlines) out[lb * NH + k].y = T(-0.5) * (zk - zm);
-        } else {
-          if (la < a.nlines) out[la * NH + k].y = T(0.5) * (zk - zm);
-          if (lb < a.nlines) out[lb * NH + k].x = T(0.5) * (zk + zm);
-        }
-      }
-    }
   }
 }
 
@@ -605,11 +514,12 @@ __device__ __forceinline__ void row_first_pass(cx<T>* v, const cx<T>* __restrict
 // butterfly NB - j (for j = 0: index R - r of this lane).  Stores A[k], B[k] for the
 // k <= N/2 = (R/3) NB this lane owns (r < R/3, and r = R/3 for j = 0) as contiguous
 // non-temporal stores.
-template <typename T, int NB, int R = 12, class Cols = PlainCols>
+// KEEP = R / 2 stores the whole half spectrum, k <= L/2; wa, wb: which of the two lines exist.
+template <typename T, int NB, int R = 12, class Cols = PlainCols, int KEEP = R / 3, bool STREAM = true>
 __device__ __forceinline__ void row_separate_store(const cx<T>* v, unsigned lane, unsigned j, vec2_t<T>* oa,
-                                                   vec2_t<T>* ob, Cols cols = Cols{}) {
+                                                   vec2_t<T>* ob, Cols cols = Cols{}, bool wa = true, bool wb = true) {
   const unsigned at = cols.at(j), step = cols.at(NB);
-  constexpr int R3 = R / 3;
+  constexpr int R3 = KEEP;
   // butterfly j of a sequence in lane j of its wave (or half-wave)
   static_assert(64 % NB == 0, "a sequence's butterflies within one wave");
   const int mlane = (int)(lane - j + (NB - j) % NB);
@@ -625,8 +535,13 @@ __device__ __forceinline__ void row_separate_store(const cx<T>* v, unsigned lane
     va.y = T(0.5) * (zk.y - zm.y);
     vb.x = T(0.5) * (zk.y + zm.y);
     vb.y = T(-0.5) * (zk.x - zm.x);
-    __builtin_nontemporal_store(va, oa + pos);
-    __builtin_nontemporal_store(vb, ob + pos);
+    if (STREAM) {
+      if (wa) __builtin_nontemporal_store(va, oa + pos);
+      if (wb) __builtin_nontemporal_store(vb, ob + pos);
+    } else {
+      if (wa) oa[pos] = va;
+      if (wb) ob[pos] = vb;
+    }
   };
   const bool j0 = j == 0;
 #pragma unroll
@@ -675,7 +590,7 @@ __global__ __launch_bounds__(P * L / 4) __attribute__((amdgpu_waves_per_eu(sizeo
   const long bps = a.nlines / (2 * P);  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
+  if (st->done) return;
 
   const int t = threadIdx.x;
   const long line0 = (blockIdx.x % bps) * (2 * P);
@@ -824,7 +739,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const long bps = a.nlines / (2 * P);  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
+  if (st->done) return;
 
   const int t = threadIdx.x;
   const long line0 = (blockIdx.x % bps) * (2 * P);
@@ -970,7 +885,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const long bps = a.nlines / 2;  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
+  if (st->done) return;
 
   const int t = threadIdx.x;
   const long la = (blockIdx.x % bps) * 2, lb = la + 1;
@@ -1476,7 +1391,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   const long bps = a.nlines / (2 * P);  // workgroups per sample
   const long sample = blockIdx.x / bps;
   DevState* st = a.st + sample;
-  if (row_idle(a, st, blockIdx.x % bps == 0)) return;
+  if (st->done) return;
 
   const int t = threadIdx.x;
   const long line0 = (blockIdx.x % bps) * (2 * P);

@@ -15,6 +15,7 @@
 #include "azb_aux_kernels.hpp"
 #include "azb_kernels.hpp"
 #include "azb_launch.hpp"
+#include "azb_seam_fft.hpp"
 
 using namespace azb;
 
@@ -203,19 +204,44 @@ int launch_row(int L, RowArgs a, long nsamples, hipStream_t st, int pdiv = 1) {
   return AZB_OK;
 }
 
+// last-axis real transforms: one wave per workgroup
 template <typename T, int L, int DIR>
-void launch_plain_row_L(PlainRowArgs a, hipStream_t st) {
-  constexpr int P = (L % 3 == 0) ? ((1536 / L) < 1 ? 1 : 1536 / L) : ((1024 / L) < 1 ? 1 : 1024 / L);
-  constexpr int NT = P * L / LenPlan<L>::E;
-  const long blocks = (a.nlines + 2 * P - 1) / (2 * P);
-  hipLaunchKernelGGL((plain_row_kernel<T, L, P, DIR>), dim3((unsigned)blocks), dim3(NT), 0, st, a);
+void launch_line_L(LineArgs a, hipStream_t st) {
+  constexpr int TS = LineCfg<T, L, DIR>::TS;
+  const dim3 blocks((unsigned)((a.nlines + 2 * TS - 1) / (2 * TS))), threads(64);
+  if constexpr (DIR < 0)
+    hipLaunchKernelGGL((line_r2c_kernel<T, L>), blocks, threads, 0, st, a);
+  else
+    hipLaunchKernelGGL((line_c2r_kernel<T, L>), blocks, threads, 0, st, a);
+}
+
+template <int DIM, int L>
+void launch_col_leray_L(LerayArgs a, hipStream_t st) {
+  constexpr int TS = LerayCfg<DIM, L>::TS;
+  hipLaunchKernelGGL((col_leray_kernel<DIM, L>), dim3((unsigned)((a.inner + TS - 1) / TS)),
+                     dim3(LerayCfg<DIM, L>::NT), 0, st, a);
 }
 
 template <typename T, int DIR>
-int launch_plain_row(int L, PlainRowArgs a, hipStream_t st) {
+int launch_line(int L, LineArgs a, hipStream_t st) {
   switch (L) {
 #define AZB_CASE(LL) \
-  case LL: launch_plain_row_L<T, LL, DIR>(a, st); break;
+  case LL: launch_line_L<T, LL, DIR>(a, st); break;
+    AZB_CASE(16) AZB_CASE(32) AZB_CASE(64) AZB_CASE(128) AZB_CASE(256) AZB_CASE(512)
+    AZB_CASE(1024) AZB_CASE(48) AZB_CASE(96) AZB_CASE(192) AZB_CASE(384) AZB_CASE(768)
+    AZB_CASE(1536)
+#undef AZB_CASE
+    default:
+      return fail(AZB_ERR_UNSUPPORTED, "FFT length " + std::to_string(L) + " not built");
+  }
+  return AZB_OK;
+}
+
+template <int DIM>
+int launch_col_leray(int L, LerayArgs a, hipStream_t st) {
+  switch (L) {
+#define AZB_CASE(LL) \
+  case LL: launch_col_leray_L<DIM, LL>(a, st); break;
     AZB_CASE(16) AZB_CASE(32) AZB_CASE(64) AZB_CASE(128) AZB_CASE(256) AZB_CASE(512)
     AZB_CASE(1024) AZB_CASE(48) AZB_CASE(96) AZB_CASE(192) AZB_CASE(384) AZB_CASE(768)
     AZB_CASE(1536)
@@ -407,6 +433,11 @@ bool stage_fused(const azb_solver* s) {
   return s->stage.width > 0 && s->plan[AZB_PROF_INV_AX0] == 0 && s->plan[AZB_PROF_FWD_AX0] == 0;
 }
 
+// One evaluation by itself pays for the column stage's idle CUs (129 workgroups at N = 1024)
+// without its gain from the next evaluation's inverse passes: 56 against 55 us FP32 for the
+// separate passes there.
+bool rhs_alone_separate(int N) { return N == 1024; }
+
 // 2D row kernel over X -> Z, both [component][line][k] with line stride ls, or in column
 // blocks of bw modes (ls = bw)
 template <typename T>
@@ -541,7 +572,7 @@ int enqueue_rhs_2d_passes(azb_solver* s, const double2* u_in, const double2* u0,
 
 int enqueue_rhs(azb_solver* s, const double2* u_in, const double2* u0, double2* out, int kmode,
                 int slot, double C, const RhsSeq& seq = {}) {
-  if (stage_fused(s))
+  if (stage_fused(s) && !(seq.lead && !seq.follow && rhs_alone_separate(s->N)))
     return s->prec == AZB_FP64 ? enqueue_rhs_2d<double>(s, u_in, u0, out, kmode, slot, C, seq)
                                : enqueue_rhs_2d<float>(s, u_in, u0, out, kmode, slot, C, seq);
   if (s->dim == 2)
@@ -792,8 +823,9 @@ int azb_dudt_noalloc(int dim, int N, int precision, azb_sv_params visc, const vo
   if (rc) return rc;
   azb_solver s;  // grid fields only: its buffers are carved out of the scratch array below
   const Layout l = setup_solver(&s, dim, N, precision, visc, 1);
-  // 2D: one sample runs the column stage, which needs its mode table in the place of Y
-  const size_t xs = round256(l.xs), ys = round256(dim == 2 ? l.ms : l.ys), zs = round256(l.zs);
+  // 2D: the column stage needs its mode table in the place of Y
+  const bool table = dim == 2 && !rhs_alone_separate(N);
+  const size_t xs = round256(l.xs), ys = round256(table ? l.ms : l.ys), zs = round256(l.zs);
   const size_t need = xs + ys + zs + round256(sizeof(DevState));
   if (need > kScratchBytes - kScratchTwBytes)
     return fail(AZB_ERR_UNSUPPORTED, std::to_string(dim) + "D N = " + std::to_string(N) + " needs " +
@@ -809,7 +841,7 @@ int azb_dudt_noalloc(int dim, int N, int precision, azb_sv_params visc, const vo
   s.Z = w + xs + ys;
   s.st = (DevState*)(w + xs + ys + zs);
   s.stream = (hipStream_t)stream;
-  if (dim == 2) {
+  if (table) {
     s.modes = (double2*)s.Y;
     launch_stage_modes(s.modes, N, visc.eps, 2 * visc.s, visc.k0, s.stream);
   }
@@ -1324,69 +1356,177 @@ int fft_work_init(void* work, int n) {
   return AZB_OK;
 }
 
-// queue one rank-dim transform; no allocation, no synchronisation
-template <typename T>
-int fft_ws_T(int dim, int n, int howmany, bool forward, void* in, void* out, void* work, hipStream_t st) {
-  if (!good_len(n)) return fail(AZB_ERR_UNSUPPORTED, "FFT length " + std::to_string(n) + " not built");
-  if (dim < 1 || dim > 3) return fail(AZB_ERR_ARG, "dim must be 1..3");
-  const void* tw = (const char*)work + kFftTwOffset;
-  const long nh = n / 2 + 1;
-  long lines = howmany;
-  for (int d = 1; d < dim; ++d) lines *= n;
+// complex passes over the leading axes d = last .. first of a (howmany, n, .., nh) array;
+// the first of them reads `in` (times scale) and writes `out`, the others run in place
+template <typename T, int DIR>
+int fft_leading(int dim, int n, int howmany, int first, const void* in, void* out, double scale, const void* work,
+                hipStream_t st) {
   ColArgs c{};
   c.nsmall = n;
-  c.tw = tw;
-  c.st = (DevState*)work;
-  PlainRowArgs p{};
-  p.nlines = lines;
-  p.tw = tw;
-  int rc;
-  // leading complex axes (axis d-2 .. 0), in place on the complex array
-  auto leading = [&](void* arr, int dir) -> int {
-    for (int ax = dim - 2; ax >= 0; --ax) {
-      long inner = nh;  // product of extents after axis ax
-      for (int d = ax + 1; d < dim - 1; ++d) inner *= n;
-      long batches = howmany;
-      for (int d = 0; d < ax; ++d) batches *= n;
-      c.in = arr;
-      c.out = arr;
-      c.nq = 1;
-      c.nk = (int)inner;
-      c.in_qs = c.out_qs = 0;
-      c.in_rs = c.out_rs = inner;
-      c.in_bs = c.out_bs = inner * n;
-      c.bps = (int)batches;  // a single device state: every batch maps to it
-      int r = dir < 0 ? launch_col_full<T, -1>(n, c, batches, st) : launch_col_full<T, +1>(n, c, batches, st);
-      if (r) return r;
-    }
-    return AZB_OK;
-  };
-  if (forward) {
-    p.in = in;
-    p.out = out;
-    if ((rc = launch_plain_row<T, -1>(n, p, st))) return rc;
-    if ((rc = leading(out, -1))) return rc;
-  } else {
-    if ((rc = leading(in, +1))) return rc;
-    p.in = in;
-    p.out = out;
-    if ((rc = launch_plain_row<T, +1>(n, p, st))) return rc;
+  c.tw = (const char*)work + kFftTwOffset;
+  c.st = (const DevState*)work;
+  c.in = in;
+  c.out = out;
+  c.scale = scale;
+  for (int ax = dim - 2; ax >= first; --ax) {
+    long inner = n / 2 + 1;  // product of extents after axis ax
+    for (int d = ax + 1; d < dim - 1; ++d) inner *= n;
+    long batches = howmany;
+    for (int d = 0; d < ax; ++d) batches *= n;
+    c.nq = 1;
+    c.nk = (int)inner;
+    c.in_rs = c.out_rs = inner;
+    c.in_bs = c.out_bs = inner * n;
+    c.bps = (int)batches;  // a single device state: every batch maps to it
+    const int rc = launch_col_full<T, DIR>(n, c, batches, st);
+    if (rc) return rc;
+    c.in = out;
+    c.scale = 1.0;
   }
+  return AZB_OK;
+}
+
+int fft_args(int dim, int n) {
+  if (!good_len(n)) return fail(AZB_ERR_UNSUPPORTED, "FFT length " + std::to_string(n) + " not built");
+  if (dim < 1 || dim > 3) return fail(AZB_ERR_ARG, "dim must be 1..3");
+  return AZB_OK;
+}
+
+template <typename T, int DIR>
+int fft_lines(int dim, int n, int howmany, const void* in, void* out, const void* work, hipStream_t st) {
+  LineArgs p{};
+  p.nlines = howmany;
+  for (int d = 1; d < dim; ++d) p.nlines *= n;
+  p.tw = (const char*)work + kFftTwOffset;
+  p.in = in;
+  p.out = out;
+  return launch_line<T, DIR>(n, p, st);
+}
+
+// queue one rank-dim transform; no allocation, no synchronisation
+template <typename T>
+int fft_r2c_T(int dim, int n, int howmany, const void* in, void* out, const void* work, hipStream_t st) {
+  int rc;
+  if ((rc = fft_args(dim, n))) return rc;
+  if ((rc = fft_lines<T, -1>(dim, n, howmany, in, out, work, st))) return rc;
+  if ((rc = fft_leading<T, -1>(dim, n, howmany, 0, out, out, 1.0, work, st))) return rc;
   HIPCHK(hipGetLastError());
   return AZB_OK;
 }
 
-// the allocating form: a temporary work area, freed after the transform finished
+// the complex array after the leading passes is tmp (in itself to overwrite the input)
 template <typename T>
-int fft_T(int dim, int n, int howmany, bool forward, void* in, void* out, hipStream_t st) {
-  if (!good_len(n)) return fail(AZB_ERR_UNSUPPORTED, "FFT length " + std::to_string(n) + " not built");
-  if (dim < 1 || dim > 3) return fail(AZB_ERR_ARG, "dim must be 1..3");
-  DevFree work;
-  HIPCHK(hipMalloc(&work.p, fft_work_bytes<T>(n)));
-  int rc = fft_work_init<T>(work.p, n);
-  if (rc) return rc;
-  if ((rc = fft_ws_T<T>(dim, n, howmany, forward, in, out, work.p, st))) return rc;
-  HIPCHK(hipStreamSynchronize(st));
+int fft_c2r_T(int dim, int n, int howmany, double scale, const void* in, void* tmp, void* out, const void* work,
+              hipStream_t st) {
+  int rc;
+  if ((rc = fft_args(dim, n))) return rc;
+  if (dim == 1 && scale != 1.0) return fail(AZB_ERR_ARG, "a scaled c2r needs dim 2 or 3");
+  if ((rc = fft_leading<T, +1>(dim, n, howmany, 0, in, tmp, scale, work, st))) return rc;
+  if ((rc = fft_lines<T, +1>(dim, n, howmany, dim > 1 ? tmp : in, out, work, st))) return rc;
+  HIPCHK(hipGetLastError());
+  return AZB_OK;
+}
+
+// Work areas of the transforms that bring none: one slot per built length and precision in
+// a file-scope array, so that a call neither allocates nor uploads.  Each GPU holds its own
+// copy for the life of the process; a slot is written once, on its first use on a device.
+constexpr int kFftLens[13] = {16, 32, 48, 64, 96, 128, 192, 256, 384, 512, 768, 1024, 1536};
+
+size_t fft_slot_offset(int n, int precision) {
+  size_t off = 0;
+  for (int p : {AZB_FP64, AZB_FP32_MIXED})
+    for (int L : kFftLens) {
+      if (p == precision && L == n) return off;
+      off += p == AZB_FP64 ? fft_work_bytes<double>(L) : fft_work_bytes<float>(L);
+    }
+  return off;
+}
+constexpr size_t kFftSlotsBytes = size_t(256) << 10;
+
+}  // namespace
+
+// Small device results of the synchronising reductions (energy spectrum, max norm): a call
+// takes one of the file-scope slots for its duration instead of allocating, or allocates
+// when all are taken or its result is longer.
+constexpr int kResultSlots = 16, kResultLen = 1024;
+static __device__ double result_slots[kResultSlots * kResultLen];
+static __device__ __align__(256) unsigned char fft_slots[kFftSlotsBytes];
+
+namespace {
+
+std::mutex g_result_mu;
+struct ResultSlots {
+  double* base = nullptr;
+  unsigned taken = 0;
+};
+std::vector<ResultSlots> g_result_slots;  // per device
+
+struct ResultSlot {
+  double* p = nullptr;
+  int dev = -1, index = -1;
+  DevFree own;
+  ResultSlot() = default;
+  ResultSlot(const ResultSlot&) = delete;
+  ResultSlot& operator=(const ResultSlot&) = delete;
+  int get(int n) {
+    HIPCHK(hipGetDevice(&dev));
+    if (n <= kResultLen) {
+      std::lock_guard<std::mutex> lock(g_result_mu);
+      if ((int)g_result_slots.size() <= dev) g_result_slots.resize(dev + 1);
+      ResultSlots& d = g_result_slots[dev];
+      if (!d.base) {
+        void* a = nullptr;
+        HIPCHK(hipGetSymbolAddress(&a, HIP_SYMBOL(result_slots)));
+        d.base = (double*)a;
+      }
+      for (int i = 0; i < kResultSlots && index < 0; ++i)
+        if (!(d.taken >> i & 1)) index = i;
+      if (index >= 0) {
+        d.taken |= 1u << index;
+        p = d.base + index * kResultLen;
+        return AZB_OK;
+      }
+    }
+    HIPCHK(hipMalloc(&own.p, sizeof(double) * n));
+    p = (double*)own.p;
+    return AZB_OK;
+  }
+  // the owner has waited for its stream, or that wait failed and the device is lost
+  ~ResultSlot() {
+    if (index < 0) return;
+    std::lock_guard<std::mutex> lock(g_result_mu);
+    g_result_slots[dev].taken &= ~(1u << index);
+  }
+};
+
+std::mutex g_fft_slots_mu;
+struct FftSlots {
+  unsigned char* base = nullptr;
+  bool ready[2][13] = {};
+};
+std::vector<FftSlots> g_fft_slots;  // per device
+
+int fft_slot(int n, int precision, void** work) {
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(g_fft_slots_mu);
+  if ((int)g_fft_slots.size() <= dev) g_fft_slots.resize(dev + 1);
+  FftSlots& d = g_fft_slots[dev];
+  if (!d.base) {
+    void* p = nullptr;
+    HIPCHK(hipGetSymbolAddress(&p, HIP_SYMBOL(fft_slots)));
+    d.base = (unsigned char*)p;
+  }
+  int i = 0;
+  while (kFftLens[i] != n) ++i;
+  void* w = d.base + fft_slot_offset(n, precision);
+  bool& ready = d.ready[precision == AZB_FP64 ? 0 : 1][i];
+  if (!ready) {
+    const int rc = precision == AZB_FP64 ? fft_work_init<double>(w, n) : fft_work_init<float>(w, n);
+    if (rc) return rc;
+    ready = true;
+  }
+  *work = w;
   return AZB_OK;
 }
 
@@ -1402,19 +1542,28 @@ int fft_check(int precision, int howmany, const void* in, const void* out, int n
 extern "C" {
 
 int azb_fft_r2c(int dim, int n, int howmany, int precision, const void* in, void* out, void* stream) {
+  void* work = nullptr;
   int rc = fft_check(precision, howmany, in, out, n);
-  if (rc) return rc;
-  hipStream_t st = (hipStream_t)stream;
-  return precision == AZB_FP64 ? fft_T<double>(dim, n, howmany, true, (void*)in, out, st)
-                               : fft_T<float>(dim, n, howmany, true, (void*)in, out, st);
+  if (rc || (rc = fft_args(dim, n)) || (rc = fft_slot(n, precision, &work))) return rc;
+  if ((rc = azb_fft_r2c_ws(dim, n, howmany, precision, in, out, work, stream))) return rc;
+  HIPCHK(hipStreamSynchronize((hipStream_t)stream));
+  return AZB_OK;
 }
 
 int azb_fft_c2r(int dim, int n, int howmany, int precision, void* in, void* out, void* stream) {
+  void* work = nullptr;
   int rc = fft_check(precision, howmany, in, out, n);
-  if (rc) return rc;
-  hipStream_t st = (hipStream_t)stream;
-  return precision == AZB_FP64 ? fft_T<double>(dim, n, howmany, false, in, out, st)
-                               : fft_T<float>(dim, n, howmany, false, in, out, st);
+  if (rc || (rc = fft_args(dim, n)) || (rc = fft_slot(n, precision, &work))) return rc;
+  if ((rc = azb_fft_c2r_ws(dim, n, howmany, precision, in, out, work, stream))) return rc;
+  HIPCHK(hipStreamSynchronize((hipStream_t)stream));
+  return AZB_OK;
+}
+
+int azb_fft_shared_work(int n, int precision, void** work) {
+  if (!work) return fail(AZB_ERR_ARG, "NULL argument");
+  if (precision != AZB_FP64 && precision != AZB_FP32_MIXED) return fail(AZB_ERR_ARG, "unknown precision");
+  if (!good_len(n)) return fail(AZB_ERR_UNSUPPORTED, "FFT length " + std::to_string(n) + " not built");
+  return fft_slot(n, precision, work);
 }
 
 size_t azb_fft_work_bytes(int n, int precision) {
@@ -1435,17 +1584,40 @@ int azb_fft_r2c_ws(int dim, int n, int howmany, int precision, const void* in, v
   if (rc) return rc;
   if (!work) return fail(AZB_ERR_ARG, "NULL work area");
   hipStream_t st = (hipStream_t)stream;
-  return precision == AZB_FP64 ? fft_ws_T<double>(dim, n, howmany, true, (void*)in, out, work, st)
-                               : fft_ws_T<float>(dim, n, howmany, true, (void*)in, out, work, st);
+  return precision == AZB_FP64 ? fft_r2c_T<double>(dim, n, howmany, in, out, work, st)
+                               : fft_r2c_T<float>(dim, n, howmany, in, out, work, st);
 }
 
 int azb_fft_c2r_ws(int dim, int n, int howmany, int precision, void* in, void* out, void* work, void* stream) {
+  return azb_fft_c2r_from(dim, n, howmany, precision, 1.0, in, in, out, work, stream);
+}
+
+int azb_fft_c2r_from(int dim, int n, int howmany, int precision, double scale, const void* in, void* tmp, void* out,
+                     void* work, void* stream) {
   int rc = fft_check(precision, howmany, in, out, n);
   if (rc) return rc;
   if (!work) return fail(AZB_ERR_ARG, "NULL work area");
+  if (!tmp && dim > 1) return fail(AZB_ERR_ARG, "NULL argument");
   hipStream_t st = (hipStream_t)stream;
-  return precision == AZB_FP64 ? fft_ws_T<double>(dim, n, howmany, false, in, out, work, st)
-                               : fft_ws_T<float>(dim, n, howmany, false, in, out, work, st);
+  return precision == AZB_FP64 ? fft_c2r_T<double>(dim, n, howmany, scale, in, tmp, out, work, st)
+                               : fft_c2r_T<float>(dim, n, howmany, scale, in, tmp, out, work, st);
+}
+
+int azb_initialize(int dim, int n, const void* u_phys, void* u_hat, void* work, void* stream) {
+  int rc = fft_check(AZB_FP64, dim, u_phys, u_hat, n);
+  if (rc) return rc;
+  if (!work) return fail(AZB_ERR_ARG, "NULL work area");
+  if (dim != 2 && dim != 3) return fail(AZB_ERR_ARG, "dim must be 2 or 3");
+  hipStream_t st = (hipStream_t)stream;
+  if ((rc = fft_lines<double, -1>(dim, n, dim, u_phys, u_hat, work, st))) return rc;
+  if ((rc = fft_leading<double, -1>(dim, n, dim, 1, u_hat, u_hat, 1.0, work, st))) return rc;
+  LerayArgs l{};
+  l.u = (double2*)u_hat;
+  l.inner = dim == 2 ? n / 2 + 1 : (long)n * (n / 2 + 1);
+  l.tw = (const char*)work + kFftTwOffset;
+  if ((rc = dim == 2 ? launch_col_leray<2>(n, l, st) : launch_col_leray<3>(n, l, st))) return rc;
+  HIPCHK(hipGetLastError());
+  return AZB_OK;
 }
 
 int azb_copy_to_padded(int dim, int N, int M, const void* in, void* out, void* stream) {
@@ -1499,14 +1671,19 @@ int azb_energy_spectrum(int dim, int N, const void* u_hat, double* spec_host, vo
   hipStream_t st = (hipStream_t)stream;
   const long nh = N / 2 + 1;
   const long nmodes = dim == 2 ? (long)N * nh : (long)N * N * nh;
-  DevFree buf;
-  HIPCHK(hipMalloc(&buf.p, sizeof(double) * nh));
-  double* d = (double*)buf.p;
-  HIPCHK(hipMemsetAsync(d, 0, sizeof(double) * nh, st));
-  long blocks = (nmodes + 255) / 256;
-  if (blocks > 2048) blocks = 2048;
-  hipLaunchKernelGGL(energy_spectrum_kernel, dim3((unsigned)blocks), dim3(256), sizeof(double) * nh, st,
-                     (const double2*)u_hat, dim, N, nmodes, d);
+  ResultSlot slot;
+  int rc = slot.get((int)nh);
+  if (rc) return rc;
+  double* d = slot.p;
+  hipLaunchKernelGGL(zero_kernel, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, st, d, (int)nh);
+  const long rows = dim == 2 ? N : (long)N * N;
+  const unsigned blocks = (unsigned)std::min<long>((rows + 3) / 4, 2048);
+  if (dim == 2)
+    hipLaunchKernelGGL(energy_spectrum_kernel<2>, dim3(blocks), dim3(256), sizeof(double) * nh, st,
+                       (const double2*)u_hat, N, nmodes, d);
+  else
+    hipLaunchKernelGGL(energy_spectrum_kernel<3>, dim3(blocks), dim3(256), sizeof(double) * nh, st,
+                       (const double2*)u_hat, N, nmodes, d);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(spec_host, d, sizeof(double) * nh, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
@@ -1525,10 +1702,11 @@ int azb_axpby(double a, const void* x, double b, void* y, long n, void* stream) 
 int azb_max_norm(const void* x, long n, double* out_host, void* stream) {
   if (!x || !out_host) return fail(AZB_ERR_ARG, "NULL argument");
   hipStream_t st = (hipStream_t)stream;
-  DevFree buf;
-  HIPCHK(hipMalloc(&buf.p, sizeof(unsigned long long)));
-  unsigned long long* d = (unsigned long long*)buf.p;
-  HIPCHK(hipMemsetAsync(d, 0, sizeof(unsigned long long), st));
+  ResultSlot slot;
+  int rc = slot.get(1);
+  if (rc) return rc;
+  unsigned long long* d = (unsigned long long*)slot.p;
+  hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, st, slot.p, 1);
   if (n > 0) {
     long blocks = (n + 255) / 256;
     if (blocks > 4096) blocks = 4096;

@@ -347,6 +347,19 @@ class Simulation:
 # ---------------------------------------------------------------------------
 # functional seams
 # ---------------------------------------------------------------------------
+def _shared_work(n: int, prec: int) -> C.c_void_p:
+    """The library's own work area for length-n transforms on the current device."""
+    work = C.c_void_p()
+    check(load().azb_fft_shared_work(n, prec, C.byref(work)))
+    return work
+
+
+def _used(t: torch.Tensor) -> None:
+    """Work on t is queued on the current stream and not waited for: its memory must not go
+    to another tensor of the stream that it was made on until that work is done."""
+    t.record_stream(torch.cuda.current_stream())
+
+
 def fft_r2c(u: torch.Tensor) -> torch.Tensor:
     """Unnormalised R2C over all but the leading (batch) axis."""
     _need("fft_r2c", u, (torch.float64, torch.float32),
@@ -357,22 +370,39 @@ def fft_r2c(u: torch.Tensor) -> torch.Tensor:
     cdt = torch.complex128 if u.dtype == torch.float64 else torch.complex64
     out = torch.empty(tuple(u.shape[:-1]) + (n // 2 + 1,), dtype=cdt, device=u.device)
     u = u.contiguous()
-    check(load().azb_fft_r2c(dim, n, u.shape[0], prec, _ptr(u), _ptr(out), _stream()))
+    pu, pout = _ptr(u), _ptr(out)
+    check(load().azb_fft_r2c_ws(dim, n, u.shape[0], prec, pu, pout, _shared_work(n, prec), _stream()))
+    _used(u)
+    return out
+
+
+_C2R_SHAPE = "(howmany, {n}, ..., {nh})"
+
+
+def _c2r_shape_ok(n: int):
+    return lambda sh: 2 <= len(sh) <= 4 and sh[0] >= 1 and all(x == n for x in sh[1:-1]) and sh[-1] == n // 2 + 1
+
+
+def _c2r(u_hat: torch.Tensor, n: int, scale: float, overwrite: bool) -> torch.Tensor:
+    """C2R of scale * u_hat (checked, contiguous); the complex passes go through a buffer of
+    their own unless u_hat may be overwritten."""
+    dim = u_hat.dim() - 1
+    prec = AZB_FP64 if u_hat.dtype == torch.complex128 else AZB_FP32_MIXED
+    rdt = torch.float64 if u_hat.dtype == torch.complex128 else torch.float32
+    pin = _ptr(u_hat)
+    out = torch.empty(tuple(u_hat.shape[:-1]) + (n,), dtype=rdt, device=u_hat.device)
+    tmp = u_hat if overwrite or dim == 1 else torch.empty_like(u_hat)
+    check(load().azb_fft_c2r_from(dim, n, u_hat.shape[0], prec, scale, pin, _ptr(tmp), _ptr(out),
+                                  _shared_work(n, prec), _stream()))
+    _used(u_hat)
     return out
 
 
 def fft_c2r(u_hat: torch.Tensor, n: int) -> torch.Tensor:
-    """Unnormalised C2R; works on a copy (the library overwrites its input)."""
-    _need("fft_c2r", u_hat, (torch.complex128, torch.complex64),
-          lambda sh: 2 <= len(sh) <= 4 and sh[0] >= 1 and all(x == n for x in sh[1:-1]) and sh[-1] == n // 2 + 1,
-          f"(howmany, {n}, ..., {n // 2 + 1})")
-    dim = u_hat.dim() - 1
-    prec = AZB_FP64 if u_hat.dtype == torch.complex128 else AZB_FP32_MIXED
-    rdt = torch.float64 if u_hat.dtype == torch.complex128 else torch.float32
-    tmp = u_hat.contiguous().clone()
-    out = torch.empty(tuple(u_hat.shape[:-1]) + (n,), dtype=rdt, device=u_hat.device)
-    check(load().azb_fft_c2r(dim, n, u_hat.shape[0], prec, _ptr(tmp), _ptr(out), _stream()))
-    return out
+    """Unnormalised C2R; u_hat is left as it is."""
+    _need("fft_c2r", u_hat, (torch.complex128, torch.complex64), _c2r_shape_ok(n),
+          _C2R_SHAPE.format(n=n, nh=n // 2 + 1))
+    return _c2r(u_hat.resolve_conj().contiguous(), n, 1.0, False)
 
 
 def leray_(u_hat: torch.Tensor) -> torch.Tensor:
@@ -385,7 +415,14 @@ def leray_(u_hat: torch.Tensor) -> torch.Tensor:
 def initialize(u_phys) -> torch.Tensor:
     """Initializer::initialize: u_hat = FFT(u) (unnormalised) then Leray, on the device."""
     u = torch.as_tensor(u_phys, dtype=torch.float64).to("cuda").contiguous()
-    return leray_(fft_r2c(u))
+    _need("initialize", u, (torch.float64,),
+          lambda sh: len(sh) in (3, 4) and sh[0] == len(sh) - 1 and len(set(sh[1:])) == 1 and sh[1] % 2 == 0,
+          "(dim, N, ..., N) with dim 2 or 3 and an even N")
+    n = u.shape[-1]
+    out = torch.empty(tuple(u.shape[:-1]) + (n // 2 + 1,), dtype=torch.complex128, device=u.device)
+    check(load().azb_initialize(u.dim() - 1, n, _ptr(u), _ptr(out), _shared_work(n, AZB_FP64), _stream()))
+    _used(u)
+    return out
 
 
 def energy_spectrum(u_hat: torch.Tensor):
@@ -444,12 +481,12 @@ def to_physical(u_hat: torch.Tensor, N_out: int | None = None) -> torch.Tensor:
     n = N if N_out is None else N_out
     if n > N:
         raise ValueError("N_out must not exceed the grid size")
-    if n == N:
-        tmp = u_hat.contiguous().clone()
-    else:
-        tmp = torch.stack([copy_from_padded(u_hat[c], n) for c in range(u_hat.shape[0])])
-    scale_(1.0 / float(N) ** dim, tmp)
-    return fft_c2r(tmp, n)
+    _need("to_physical", u_hat, (torch.complex128,))
+    u_hat = u_hat.resolve_conj()
+    if n < N:
+        u_hat = torch.stack([copy_from_padded(u_hat[c], n) for c in range(u_hat.shape[0])])
+    _need("to_physical", u_hat, (torch.complex128,), _c2r_shape_ok(n), _C2R_SHAPE.format(n=n, nh=n // 2 + 1))
+    return _c2r(u_hat.contiguous(), n, 1.0 / float(N) ** dim, n < N)
 
 
 def axpby_(a: float, x: torch.Tensor, b: float, y: torch.Tensor) -> torch.Tensor:

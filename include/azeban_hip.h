@@ -223,6 +223,22 @@ int azb_fft_r2c_ws(int dim, int n, int howmany, int precision, const void* in, v
 int azb_fft_c2r_ws(int dim, int n, int howmany, int precision, void* in, void* out, void* work,
                    void* stream);
 
+/* The work area that azb_fft_r2c / azb_fft_c2r themselves use for (n, precision) on the
+ * current device: held for the life of the process, shared by every caller, never freed by
+ * one.  Its first use on a device uploads the tables (synchronising, not under capture);
+ * later calls only return the pointer. */
+int azb_fft_shared_work(int n, int precision, void** work);
+/* azb_fft_c2r_ws of scale times the input, which is left as it is: the complex passes go
+ * through tmp, an array of the input's size (unused for dim 1, where scale must be 1;
+ * tmp = in overwrites the input). */
+int azb_fft_c2r_from(int dim, int n, int howmany, int precision, double scale, const void* in, void* tmp, void* out,
+                     void* work, void* stream);
+/* Initializer::initialize on the device (include/azeban/init/initializer.hpp:68-75): the
+ * unnormalised transform of dim real components (dim, n, .., n) and their Leray projection
+ * into u_hat (dim, n, .., n/2+1); work is an FP64 work area of length n.  Queued on
+ * `stream`; the same as azb_fft_r2c_ws then azb_leray to round-off. */
+int azb_initialize(int dim, int n, const void* u_phys, void* u_hat, void* work, void* stream);
+
 /* One component N -> M zero padding, copy_to_padded
  * (src/azeban/operations/copy_to_padded.cpp:301-328,
  *  include/azeban/operations/copy_to_padded_functions.hpp:11-63). */
