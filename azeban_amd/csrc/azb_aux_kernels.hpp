@@ -21,24 +21,39 @@ __global__ void step_prologue_fixed(DevState* st_all, double max_dt) {
   }
 }
 
-// device-driven loop: a step past t_end does nothing (done = 1)
-__global__ void step_prologue_loop(DevState* st_all) {
+// Control of the device-driven loop between steps: `end` advances the time of the step that
+// was run, `begin` decides whether the next one runs (a step past t_end does nothing, done =
+// 1), sets its clamp and clears the max|u| bins.
+__global__ void step_control_loop(DevState* st_all, int end, int begin) {
   DevState* st = st_all + blockIdx.x;
   const int t = threadIdx.x;
-  const bool go = st->time < st->t_end;
-  for (int e = t; e < 4 * kBins; e += blockDim.x) (&st->umax_bins[0][0])[e] = 0ull;
   if (t == 0) {
-    st->done = go ? 0 : 1;
-    if (go) st->max_dt = fmin(st->t_end - st->time, st->max_dt_visc);
+    double time = st->time;
+    if (end && !st->done) {
+      time += st->dt;
+      st->time = time;
+      st->steps += 1;
+    }
+    if (begin) {
+      const bool go = time < st->t_end;
+      st->done = go ? 0 : 1;
+      if (go) st->max_dt = fmin(st->t_end - time, st->max_dt_visc);
+    }
   }
+  if (begin)
+    for (int e = t; e < 4 * kBins; e += blockDim.x) (&st->umax_bins[0][0])[e] = 0ull;
 }
 
-__global__ void step_epilogue_loop(DevState* st_all) {
-  DevState* st = st_all + blockIdx.x;
-  if (threadIdx.x == 0 && !st->done) {
-    st->time += st->dt;
-    st->steps += 1;
-  }
+// start the device-driven loop of every sample at one time and target
+__global__ void loop_set_all(DevState* st_all, int nsamples, double time, double t_end, double max_dt_visc) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nsamples) return;
+  DevState* st = st_all + i;
+  st->time = time;
+  st->t_end = t_end;
+  st->max_dt_visc = max_dt_visc;
+  st->done = 0;
+  st->steps = 0;
 }
 
 // (re)start the device-driven loop of one sample: its time, target and step count
@@ -53,7 +68,8 @@ __global__ void loop_set_sample(DevState* st_all, int sample, double time, doubl
 }
 
 // reduce one slot's bins: u_max = max / M^d; stage 1 also sets dt = min(C/(N u_max), max_dt)
-__global__ void finalize_umax(DevState* st_all, int slot, int set_dt, double Md, double C, double N) {
+// (dt_out: also there, for the first sample)
+__global__ void finalize_umax(DevState* st_all, int slot, int set_dt, double Md, double C, double N, double* dt_out) {
   DevState* st = st_all + blockIdx.x;
   if (st->done) return;
   const int t = threadIdx.x;  // 64 threads
@@ -62,7 +78,11 @@ __global__ void finalize_umax(DevState* st_all, int slot, int set_dt, double Md,
   if (t == 0) {
     const double um = v / Md;
     st->u_max = um;
-    if (set_dt) st->dt = fmin(C / (N * um), st->max_dt);
+    if (set_dt) {
+      const double dt = fmin(C / (N * um), st->max_dt);
+      st->dt = dt;
+      if (dt_out && blockIdx.x == 0) *dt_out = dt;
+    }
   }
 }
 

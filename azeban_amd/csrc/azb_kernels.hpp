@@ -265,10 +265,11 @@ struct KArgs {
   double eps, s2, k0;    // SmoothCutoff1D with s2 = 2s
   int mode;              // KMode: the kernel's MODE
   DevState* st;          // one per sample
-  // fold = 1 (2D): the max|u| reduction of this RHS runs here instead of in a kernel
-  // of its own: u_max = max(bins[slot]) / Md, at stage 1 dt = min(C / (Nd u_max), max_dt)
+  // fold = 1: the max|u| reduction of this RHS runs here instead of in a kernel of its own:
+  // u_max = max(bins[slot]) / Md, at stage 1 dt = min(C / (Nd u_max), max_dt)
   int fold, slot;
   double Md, C, Nd;
+  double* dt_out;  // host-visible copy of the first sample's dt (NULL: none)
 };
 
 __device__ __forceinline__ double sv_eval(double k, double eps, double s2, double k0) {
@@ -389,7 +390,10 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
     dt = MODE == K_RK1 ? fmin(a.C / (a.Nd * um), st->max_dt) : st->dt;
     if (first && threadIdx.x == 0) {
       st->u_max = um;
-      if (MODE == K_RK1) st->dt = dt;
+      if (MODE == K_RK1) {
+        st->dt = dt;
+        if (a.dt_out && sample == 0) *a.dt_out = dt;
+      }
     }
   } else {
     dt = st->dt;

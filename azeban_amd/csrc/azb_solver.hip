@@ -57,6 +57,9 @@ bool good_len(int L) {
   }
 }
 
+// widest column tile of the passes at length L (azb::col_ts at run time)
+int col_ts_of(size_t tsize, int L) { return std::max(1, 6144 * (8 / (int)tsize) / L); }
+
 // line pairs per workgroup of the fused row kernel
 int row_p(int L) {
   int p = 1536 / L;
@@ -283,6 +286,9 @@ struct azb_solver {
   // radix plan per column-pass family (ColPlan index; the row and k-space entries are 0)
   int plan[AZB_PROF_FAMILIES] = {0, 0, 0, 0, 0, 0};
   StageShape stage{0, 0};  // 2D column stage; width 0: separate passes
+  double* dt_host = nullptr;  // pinned, written by the kernels of a fixed step that reports its dt
+  double* dt_out = nullptr;   // dt_host while such a step is queued
+  DevState* read_host = nullptr;  // pinned mirror of the device state (blocking reads)
   DevState* probe_host = nullptr;  // pinned mirror of the device state (non-blocking probes)
   hipEvent_t probe_ev = nullptr;
   // per-kernel-family hipEvent timing (off unless enabled)
@@ -394,8 +400,17 @@ int enqueue_rhs_3d(azb_solver* s, const double2* u_in, const double2* u0, double
   }
   const double Md = std::pow((double)M, 3);
   KArgs k{};
-  hipLaunchKernelGGL(finalize_umax, dim3((unsigned)S), dim3(64), 0, st, s->st, slot, kmode == K_RK1 ? 1 : 0, Md, C,
-                     (double)N);
+  // small grids reduce max|u| in the k-space kernel (a launch of 4 us less per evaluation);
+  // large ones do not have each of a million waves read the bins
+  k.fold = N <= 128 ? 1 : 0;
+  k.slot = slot;
+  k.Md = Md;
+  k.C = C;
+  k.Nd = (double)N;
+  k.dt_out = s->dt_out;
+  if (!k.fold)
+    hipLaunchKernelGGL(finalize_umax, dim3((unsigned)S), dim3(64), 0, st, s->st, slot, kmode == K_RK1 ? 1 : 0, Md, C,
+                       (double)N, s->dt_out);
   k.bh = s->Y;
   k.u_in = u_in;
   k.u0 = u0;
@@ -479,6 +494,7 @@ int enqueue_rhs_2d(azb_solver* s, const double2* u_in, const double2* u0, double
     g.tw_i = (const cx<T>*)s->tw + col_ptab_offset(0, +1);
   }
   g.st = s->st;
+  g.dt_out = s->dt_out;
   g.slot = slot;
   g.clear = -1;
   const std::string not_built = "column length " + std::to_string(M) + " not built";
@@ -548,6 +564,7 @@ int enqueue_rhs_2d_passes(azb_solver* s, const double2* u_in, const double2* u0,
   k.Md = std::pow((double)M, 2);
   k.C = C;
   k.Nd = (double)N;
+  k.dt_out = s->dt_out;
   k.bh = s->Y;
   k.u_in = u_in;
   k.u0 = u0;
@@ -611,6 +628,10 @@ int check_solver_args(int dim, int N, int M, int n_vars, int precision, int nsam
   return AZB_OK;
 }
 
+size_t round256(size_t b) { return (b + 255) / 256 * 256; }
+
+size_t bhat_bytes_2d(const azb_solver* s) { return (size_t)s->S * 2 * s->tsize * 3 * (size_t)s->N * s->nhp; }
+
 // bytes of the intermediates X, Y, Z and of one RK stage buffer for S samples
 struct Layout {
   size_t xs, ys, zs, us;
@@ -631,6 +652,18 @@ Layout setup_solver(azb_solver* s, int dim, int N, int precision, azb_sv_params 
   // 3D: the 12-values-per-thread row kernel with 192-thread workgroups
   s->pdiv = dim == 3 ? 2 : 1;
   s->tsize = precision == AZB_FP64 ? 8 : 4;
+  // 3D column tiles of one 128-byte line at working precision (the narrowest built where
+  // that is more than a quarter of the widest), which waste fewer lanes on the last tile of
+  // N/2+1 columns than the widest and give small grids more workgroups: RHS 64^3 74.7 ->
+  // 73.2 us FP64 and 68 -> 60 FP32, 128^3 266 -> 235 FP32, 256^3 2584 -> 2511 FP64 and 1630
+  // -> 1593 FP32.  The FP32 first pass at N = 256 reads the FP64 state and stays at the
+  // widest (170 against 186 us).
+  if (dim == 3) {
+    int div = 1;
+    while (div < 4 && col_ts_of(s->tsize, M) / div * 2 * (int)s->tsize > 128) div *= 2;
+    for (int f : {AZB_PROF_INV_AX0, AZB_PROF_INV_AX1, AZB_PROF_FWD_AX1, AZB_PROF_FWD_AX0}) s->tsdiv[f] = div;
+    if (precision != AZB_FP64 && N == 256) s->tsdiv[AZB_PROF_INV_AX0] = 1;
+  }
   const size_t cs = 2 * s->tsize;  // complex at working precision
   const long nh = s->nh;
   s->nhp = (nh + 15) / 16 * 16;
@@ -645,10 +678,11 @@ Layout setup_solver(azb_solver* s, int dim, int N, int precision, azb_sv_params 
   } else {
     s->nmodes = (long)N * nh;
     l.xs = S * cs * 2 * (size_t)M * hp;
-    l.ys = S * cs * 3 * (size_t)N * hp;
     l.zs = S * cs * 3 * (size_t)M * hp;
     s->stage = stage_shape((int)s->tsize, M, nsamples);
     if (s->stage.width) l.ms = sizeof(double2) * s->nmodes;
+    // B_hat exists only between separate passes
+    if (!s->stage.width || rhs_alone_separate(N)) l.ys = bhat_bytes_2d(s);
   }
   l.us = S * sizeof(double2) * (size_t)dim * s->nmodes;
   if (s->stage.width)  // in column blocks
@@ -656,7 +690,6 @@ Layout setup_solver(azb_solver* s, int dim, int N, int precision, azb_sv_params 
   return l;
 }
 
-size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 // ---------------------------------------------------------------------------
 // Scratch of the no-allocation RHS (azb_dudt_noalloc): the twiddle tables of every
@@ -738,12 +771,14 @@ int azb_create_batch(int dim, int N, int M, int n_vars, int precision, azb_sv_pa
     azb_destroy(s);
     return fail(code, m);
   };
-  if (hipMalloc(&s->X, xs) != hipSuccess || hipMalloc(&s->Y, ys) != hipSuccess ||
-      hipMalloc(&s->Z, zs) != hipSuccess || (ms && hipMalloc((void**)&s->modes, ms) != hipSuccess) || hipMalloc((void**)&s->u1, us) != hipSuccess ||
+  // the mode table lies behind the first stage buffer, in its allocation
+  const size_t modes_at = round256(us);
+  if (hipMalloc(&s->X, xs) != hipSuccess || (ys && hipMalloc(&s->Y, ys) != hipSuccess) ||
+      hipMalloc(&s->Z, zs) != hipSuccess || hipMalloc((void**)&s->u1, modes_at + ms) != hipSuccess ||
       hipMalloc((void**)&s->u2, us) != hipSuccess ||
       hipMalloc((void**)&s->st, S * sizeof(DevState)) != hipSuccess)
     return cleanup(AZB_ERR_ALLOC, "device allocation of the solver workspace failed");
-  s->bytes = xs + ys + zs + 2 * us + ms + S * sizeof(DevState);
+  s->bytes = xs + ys + zs + modes_at + ms + us + S * sizeof(DevState);
   rc = precision == AZB_FP64 ? make_twiddles<double>(s->M, &s->tw) : make_twiddles<float>(s->M, &s->tw);
   if (rc) {
     std::string m = g_err;
@@ -753,7 +788,8 @@ int azb_create_batch(int dim, int N, int M, int n_vars, int precision, azb_sv_pa
   std::vector<DevState> h(S);
   if (hipMemcpy(s->st, h.data(), S * sizeof(DevState), hipMemcpyHostToDevice) != hipSuccess)
     return cleanup(AZB_ERR_HIP, "hipMemcpy of the device state failed");
-  if (s->modes) {
+  if (ms) {
+    s->modes = (double2*)((char*)s->u1 + modes_at);
     launch_stage_modes(s->modes, N, visc.eps, 2 * visc.s, visc.k0, s->stream);
     if (hipGetLastError() != hipSuccess) return cleanup(AZB_ERR_HIP, "launch of the mode table kernel failed");
   }
@@ -776,8 +812,8 @@ size_t azb_bytes_estimate(int dim, int N, int precision, int nsamples) {
     ws = cs * (6 * M * N * hp + std::max(3 * M * M * hp, 6 * (size_t)N * N * hp) + 6 * M * M * hp);
     us = sizeof(double2) * 3 * (size_t)N * N * nh;
   } else {
-    ws = cs * (2 * M * hp + 3 * (size_t)N * hp + 3 * M * hp);
     const size_t w = stage_shape(precision == AZB_FP64 ? 8 : 4, (int)M, nsamples).width;
+    ws = cs * (2 * M * hp + (w && !rhs_alone_separate(N) ? 0 : 3 * (size_t)N * hp) + 3 * M * hp);
     us = sizeof(double2) * 2 * (size_t)N * (w ? (nh + w - 1) / w * w : nh);
     ms = w ? sizeof(double2) * (size_t)N * nh : 0;
   }
@@ -790,11 +826,12 @@ int azb_destroy(azb_solver* s) {
   (void)hipFree(s->X);
   (void)hipFree(s->Y);
   (void)hipFree(s->Z);
-  (void)hipFree(s->modes);
   (void)hipFree(s->u1);
   (void)hipFree(s->u2);
   (void)hipFree(s->st);
   (void)hipFree(s->tw);
+  if (s->dt_host) (void)hipHostFree(s->dt_host);
+  if (s->read_host) (void)hipHostFree(s->read_host);
   if (s->probe_host) (void)hipHostFree(s->probe_host);
   if (s->probe_ev) (void)hipEventDestroy(s->probe_ev);
   for (auto& e : s->prof_ev) {
@@ -868,12 +905,16 @@ int azb_dt(azb_solver* s, double C, double* dt_host) {
 
 int azb_rk3_step(azb_solver* s, void* u_hat, double max_dt, double C, double* dt_host) {
   if (!s || !u_hat) return fail(AZB_ERR_ARG, "NULL argument");
+  if (dt_host && !s->dt_host) HIPCHK(hipHostMalloc((void**)&s->dt_host, sizeof(double), hipHostMallocDefault));
   hipLaunchKernelGGL(step_prologue_fixed, dim3(s->S), dim3(256), 0, s->stream, s->st, max_dt);
+  // the kernel that takes dt also stores it where the host reads it: no copy to wait for
+  s->dt_out = dt_host ? s->dt_host : nullptr;
   int rc = enqueue_rk3_stages(s, (double2*)u_hat, C);
+  s->dt_out = nullptr;
   if (rc) return rc;
   if (dt_host) {
-    HIPCHK(hipMemcpyAsync(dt_host, &s->st->dt, sizeof(double), hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
+    *dt_host = *s->dt_host;
   }
   return AZB_OK;
 }
@@ -918,23 +959,26 @@ int azb_enqueue_steps(azb_solver* s, void* u_hat, int nsteps) {
   const bool fused = stage_fused(s);
   for (int i = 0; i < nsteps; ++i) {
     const bool lead = !fused || i == 0;
-    if (lead) hipLaunchKernelGGL(step_prologue_loop, dim3(s->S), dim3(256), 0, s->stream, s->st);
+    // ends the previous step of this call, if it was not the column stage's, and starts this one
+    if (lead) hipLaunchKernelGGL(step_control_loop, dim3(s->S), dim3(256), 0, s->stream, s->st, i > 0 ? 1 : 0, 1);
     int rc = enqueue_rk3_stages(s, (double2*)u_hat, s->loop_C, lead, i + 1 < nsteps, fused);
     if (rc) return rc;
-    if (!fused) hipLaunchKernelGGL(step_epilogue_loop, dim3(s->S), dim3(64), 0, s->stream, s->st);
   }
+  if (!fused && nsteps > 0)
+    hipLaunchKernelGGL(step_control_loop, dim3(s->S), dim3(64), 0, s->stream, s->st, 1, 0);
   HIPCHK(hipGetLastError());
   return AZB_OK;
 }
 
 int azb_loop_read(azb_solver* s, double* times_host, int* steps_host) {
   if (!s) return fail(AZB_ERR_ARG, "NULL solver");
-  std::vector<DevState> h(s->S);
-  HIPCHK(hipMemcpyAsync(h.data(), s->st, s->S * sizeof(DevState), hipMemcpyDeviceToHost, s->stream));
+  if (!s->read_host)
+    HIPCHK(hipHostMalloc((void**)&s->read_host, s->S * sizeof(DevState), hipHostMallocDefault));
+  HIPCHK(hipMemcpyAsync(s->read_host, s->st, s->S * sizeof(DevState), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
   for (int i = 0; i < s->S; ++i) {
-    if (times_host) times_host[i] = h[i].time;
-    if (steps_host) steps_host[i] = h[i].steps;
+    if (times_host) times_host[i] = s->read_host[i].time;
+    if (steps_host) steps_host[i] = s->read_host[i].steps;
   }
   return AZB_OK;
 }
@@ -981,10 +1025,15 @@ int azb_simulate_until(azb_solver* s, void* u_hat, double t_end, double C, doubl
                        int max_steps, int chunk, int* steps_out) {
   if (!s || !u_hat || !time_inout) return fail(AZB_ERR_ARG, "NULL argument");
   if (chunk <= 0) chunk = 8;
-  std::vector<double> t0(s->S, *time_inout), times(s->S);
+  std::vector<double> times(s->S);
   std::vector<int> steps(s->S);
-  int rc = azb_loop_begin(s, t_end, C, t0.data());
-  if (rc) return rc;
+  int rc;
+  // azb_loop_begin without its upload and wait: every sample starts at the same time
+  const double pi = 3.14159265358979323846;
+  s->loop_C = C;
+  s->loop_begun = true;
+  hipLaunchKernelGGL(loop_set_all, dim3((unsigned)((s->S + 63) / 64)), dim3(64), 0, s->stream, s->st, s->S, *time_inout,
+                     t_end, C * 2. / (s->visc.eps * ((pi * s->N) * (pi * s->N))));
   int taken = 0;
   while (true) {
     int n = chunk;
@@ -1203,6 +1252,11 @@ int azb_set_plans(azb_solver* s, const int* plans) {
     if (plans[f] < 0 || plans[f] >= (col ? n : 1))
       return fail(AZB_ERR_ARG, "radix plan " + std::to_string(plans[f]) + " of family " + std::to_string(f) +
                                    " outside [0, " + std::to_string(col ? n : 1) + ")");
+  }
+  if (s->dim == 2 && !s->Y && (plans[AZB_PROF_INV_AX0] || plans[AZB_PROF_FWD_AX0])) {
+    // these plans run the separate passes
+    HIPCHK(hipMalloc(&s->Y, bhat_bytes_2d(s)));
+    s->bytes += bhat_bytes_2d(s);
   }
   for (int f = 0; f < AZB_PROF_FAMILIES; ++f) s->plan[f] = plans[f];
   return AZB_OK;

@@ -141,6 +141,7 @@ struct StageArgs {
   int mode, slot;       // KMode, or K_LEAD: only the inverse transforms, of u_in
   int clear;    // max|u| slot whose bins the next row kernel fills: cleared here (-1: none)
   int advance;  // last stage of a step of the device-driven loop: time += dt, ++steps
+  double* dt_out;  // host-visible copy of the first sample's dt (NULL: none)
 };
 
 // First and remaining radices of a plan
@@ -216,7 +217,10 @@ __global__ __launch_bounds__((StageCfg<T, L, TS, F>::NT)) __attribute__((amdgpu_
     dt = a.mode == K_RK1 ? fmin(a.C / (a.Nd * um), st->max_dt) : st->dt;
     if (first && t == 0) {
       st->u_max = um;
-      if (a.mode == K_RK1) st->dt = dt;
+      if (a.mode == K_RK1) {
+        st->dt = dt;
+        if (a.dt_out && sample == 0) *a.dt_out = dt;
+      }
       if (a.advance) {
         st->time += dt;
         st->steps += 1;
