@@ -15,7 +15,7 @@ void launch_row4_P(const RowArgs& a, long nsamples, hipStream_t st) {
   hipLaunchKernelGGL((euler_row4_kernel<T, L, P>), dim3((unsigned)blocks), dim3(Row4Cfg<T, L, P>::NT), 0, st, a);
 }
 
-// pdiv in {1, 2}: where the row-4 kernel runs (3D L = 96; FP32 at L = 192) it
+// pdiv in {1, 2}: where the row-4 kernel runs (3D FP32 at L = 96 and 192) it
 // takes P0 = 1536/L line pairs per workgroup or half of that; every other kernel
 // has one line-pair tile
 template <typename T, int L, int DIM>
@@ -33,14 +33,14 @@ void launch_row_L(const RowArgs& a, long nsamples, hipStream_t st, int pdiv) {
     const long blocks = a.nlines / 2 * nsamples;
     hipLaunchKernelGGL((euler_row6_kernel<T>), dim3((unsigned)blocks), dim3(Row6Cfg::NT), 0, st, a);
     (void)pdiv;
-  } else if constexpr (DIM == 3 && (L == 96 || (L == 192 && sizeof(T) == 4))) {
+  } else if constexpr (DIM == 3 && (L == 96 || L == 192) && sizeof(T) == 4) {
     constexpr int P0 = 1536 / L, P1 = P0 / 2;
     if (pdiv == 2)
       launch_row4_P<T, L, P1>(a, nsamples, st);
     else
       launch_row4_P<T, L, P0>(a, nsamples, st);
   } else if constexpr (DIM == 3) {
-    // 3D at L = 384, and FP64 at L = 192: 768/L line pairs per workgroup with a
+    // 3D at L = 384, and FP64 at L = 192 and 96: 768/L line pairs per workgroup with a
     // single forward round, whatever pdiv says (one plan per precision and size)
     const long blocks = a.nlines / (2 * Row6pCfg<L>::P) * nsamples;
     hipLaunchKernelGGL((euler_row6p_kernel<T, L>), dim3((unsigned)blocks), dim3(Row6pCfg<L>::NT), 0, st, a);
@@ -66,7 +66,10 @@ void launch_row_L(const RowArgs& a, long nsamples, hipStream_t st, int pdiv) {
 template <typename T, int DIM>
 int launch_row_T(int L, const RowArgs& a, long nsamples, hipStream_t st, int pdiv) {
   switch (L) {
-    case 96: launch_row_L<T, 96, DIM>(a, nsamples, st, pdiv); return 0;
+    case 96:
+      if (DIM == 3 && sizeof(T) == 8 && a.nlines % 16 != 0) return 2;  // eight line pairs per workgroup
+      launch_row_L<T, 96, DIM>(a, nsamples, st, pdiv);
+      return 0;
     case 192:
       if (DIM == 3 && sizeof(T) == 8 && a.nlines % 8 != 0) return 2;  // four line pairs per workgroup
       launch_row_L<T, 192, DIM>(a, nsamples, st, pdiv);

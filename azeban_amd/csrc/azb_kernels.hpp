@@ -124,18 +124,26 @@ __device__ __forceinline__ unsigned xcd_contiguous(unsigned b, unsigned nb) {
   return x * q + (x < r ? x : r) + i;
 }
 
+// Threads of a column pass: LenPlan's E values per thread, or half of that (and a short
+// last round where a radix does not divide it) at L = 96, whose passes run with one or two
+// waves per SIMD and take one wave's chain of instructions (64^3 FP64: forward axis 1 15.3 ->
+// 12.9 us, inverse axis 0 11.1 -> 10.4, axis 1 8.0 -> 7.0; same rounding).
+template <int L, int MODE>
+constexpr int col_values() { return L == 96 && MODE != COL_FULL ? LenPlan<L>::E / 2 : LenPlan<L>::E; }
+
 template <typename Tin, typename Tout, typename T, int L, int TS, int DIR, int MODE, int V = 0>
-__global__ __launch_bounds__(TS * L / LenPlan<L>::E, (sizeof(T) == 4 ? 4 : (L == 768 || L == 384 ? 3 : 2))) void col_fft_kernel(ColArgs a) {
-  using LP = LenPlan<L>;
+__global__ __launch_bounds__((TS * L / col_values<L, MODE>()), (sizeof(T) == 4 ? 4 : (L == 768 || L == 384 ? 3 : 2))) void col_fft_kernel(ColArgs a) {
   using PP = typename ColPlan<L, V>::P;
-  constexpr int E = LP::E;
-  constexpr int NT = TS * L / E;
+  constexpr int NT = TS * L / col_values<L, MODE>();
   // exchange in one barrier pair unless the interleaved buffer would exceed 64 KB
   constexpr bool SPLIT = TS * L * 2 * (int)sizeof(T) > 65536;
   // FP32 at L = 768 in the RHS: twiddles from the plan's per-pass table (the
   // launcher points a.tw at it), one base address per butterfly and 16-byte loads
   constexpr bool PT = sizeof(T) == 4 && L == 768 && MODE != COL_FULL;
-  using F = BlockFFT2<T, L, TS, NT, DIR, SPLIT, 1, MAP_STD, MAP_STD, false, 1, 0u, 0, 0u, void, PT>;
+  using FB = BlockFFT2<T, L, TS, TS * L / LenPlan<L>::E, DIR, SPLIT, 1, MAP_STD, MAP_STD, false, 1, 0u, 0, 0u, void, PT>;
+  using FC = ColFFT<T, L, TS, NT, DIR, SPLIT, ColLayout<TS, 0>, PT>;
+  using F = std::conditional_t<col_values<L, MODE>() == LenPlan<L>::E, FB, FC>;
+  constexpr int E = FC::values(PP{});
   constexpr int R0 = first_radix(PP{});
   constexpr int RL = last_radix(PP{});
   __shared__ T lds[F::lds_words];
@@ -1340,17 +1348,18 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
 }
 
 // ---------------------------------------------------------------------------
-// 3D row kernel at L = 384 and 192 (N = 256, 128) with one forward round:
+// 3D row kernel at L = 384, 192 and 96 (N = 256, 128, 64) with one forward round:
 // P = 768/L line pairs per 192-thread workgroup.  The inverse is the row-4
 // kernel's (3P packed sequences, 12 values per thread, plans 12.2.4.4 / 12.4.4;
 // at L = 384 its two middle passes run in half-waves, each sequence in its own
 // half-wave, so two of the three exchanges need no workgroup barrier); all six
 // products of a pair are formed at once and one 6P-sequence forward transform
 // (24 values per thread, plans 4.4.24 / 4.2.24, exchanges in real/imaginary
-// halves) replaces two rounds of 3P.  (At L = 96 the per-sequence pad
-// slots of 24 sequences would not leave room for four workgroups per CU; the
-// row-4 kernel stays there, and for FP32 at L = 192, where its four waves per
-// SIMD measured faster.)  The radix-24 last
+// halves) replaces two rounds of 3P.  FP64 at L = 96 (P = 8, plans 12.2.4 / 4.24)
+// too: one forward exchange instead of four, 19.4 -> 17.2 us at 64^3, whose 576
+// workgroups are resident together although three, not four, fit a CU.  (FP32
+// at L = 96 and 192 keeps the row-4 kernel, whose four waves per SIMD measured
+// faster at 192.)  The radix-24 last
 // pass keeps butterfly j of a sequence in lane j of an L/24-lane group, so the
 // separation of each packed spectrum stays within a wave.
 // ---------------------------------------------------------------------------
@@ -1358,6 +1367,7 @@ template <int L>
 struct Row6pPlan;
 template <> struct Row6pPlan<384> { using Inv = Plan<12, 2, 4, 4>; using Fwd = Plan<4, 4, 24>; };
 template <> struct Row6pPlan<192> { using Inv = Plan<12, 4, 4>; using Fwd = Plan<4, 2, 24>; };
+template <> struct Row6pPlan<96> { using Inv = Plan<12, 2, 4>; using Fwd = Plan<4, 24>; };
 
 template <int L_>
 struct Row6pCfg {
@@ -1389,7 +1399,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
                        C::template fwd_pade<T>()>;
   static_assert(FI::E == 12 && FF::E == 24, "thread layout");
   constexpr int XWORDS = FI::lds_words > FF::lds_words ? FI::lds_words : FF::lds_words;
-  static_assert(4 * (XWORDS * (int)sizeof(T) + 3 * 8) <= 163840, "four workgroups per CU");
+  static_assert((L == 96 ? 3 : 4) * (XWORDS * (int)sizeof(T) + 3 * 8) <= 163840, "workgroups per CU");
   __shared__ T X[XWORDS];
   __shared__ double red[NT / 64];
   const long bps = a.nlines / (2 * P);  // workgroups per sample

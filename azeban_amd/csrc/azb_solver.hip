@@ -125,13 +125,12 @@ int make_twiddles(int L, void** out) {
 // ---------------------------------------------------------------------------
 template <typename Tin, typename Tout, typename T, int L, int TS, int DIR, int MODE, int V = 0>
 void launch_col_TS(ColArgs a, long batches, hipStream_t st) {
-  constexpr int E = LenPlan<L>::E;
   // the FP32 768-point passes of the RHS read their plan's per-pass table
   if constexpr (sizeof(T) == 4 && L == 768 && MODE != COL_FULL) a.tw = (const cx<T>*)a.tw + col_ptab_offset(V, DIR);
   a.ktiles = (a.nk + TS - 1) / TS;
   const long blocks = batches * a.nq * a.ktiles;
   hipLaunchKernelGGL((col_fft_kernel<Tin, Tout, T, L, TS, DIR, MODE, V>), dim3((unsigned)blocks),
-                     dim3(TS * L / E), 0, st, a);
+                     dim3(TS * L / (col_values<L, MODE>())), 0, st, a);
 }
 
 // tsdiv in {1, 2, 4} selects tiles of TS0, TS0/2 or TS0/4 columns, TS0 being one

@@ -12,114 +12,6 @@
 
 namespace azb {
 
-// LDS layout of the exchanges: element (s, pos) at pos*TSt + s with PAD pad slots after
-// every 8 positions (the radix-8 first passes write 8 consecutive positions per
-// butterfly; the pad spreads consecutive butterflies over the banks).
-template <int TSt, int PAD>
-struct ColLayout {
-  __device__ __forceinline__ static unsigned at(unsigned s, unsigned pos) {
-    return pos * (unsigned)TSt + s + (pos >> 3) * (unsigned)PAD;
-  }
-  static constexpr bool linear(int D) { return D % 8 == 0; }
-  static constexpr unsigned delta(int D) { return D * TSt + D / 8 * PAD; }
-  static constexpr int elems(int L) { return L * TSt + L / 8 * PAD; }
-};
-
-// Stockham passes of TSt sequences of length L over NT threads, sequences fastest across
-// threads (s = g % TSt, j = g / TSt, g = t + NT b).  A pass whose butterflies do not fill
-// the threads evenly leaves the last round's surplus threads idle, so any radix works
-// with any thread count.  The arithmetic per butterfly is BlockFFT2's.
-template <typename T, int L, int TSt, int NT, int DIR, bool SPLIT, class LAY, bool PTAB>
-struct ColFFT {
-  static_assert(NT % TSt == 0, "a thread keeps its sequence");
-  static constexpr unsigned JS = NT / TSt;
-  template <int R>
-  static constexpr int rounds() { return (TSt * (L / R) + NT - 1) / NT; }
-  // round b of a radix-R pass: whether thread t has a butterfly there
-  template <int R>
-  __device__ __forceinline__ static bool on(unsigned j, int b) {
-    return (b + 1) * NT <= TSt * (L / R) || j + JS * b < (unsigned)(L / R);
-  }
-  using twptr = const __attribute__((address_space(1))) cx<T>*;
-
-  template <int Ns, int R>
-  __device__ __forceinline__ static void butterflies(cx<T>* v, unsigned t_in, const cx<T>* tw_in) {
-    // opaque copies keep each pass's twiddle loads and indices inside the pass
-    twptr tw = (twptr)tw_in;
-    asm volatile("" : "+s"(tw));
-    unsigned t = t_in;
-    asm volatile("" : "+v"(t));
-    const unsigned j = t / (unsigned)TSt;
-#pragma unroll
-    for (int b = 0; b < rounds<R>(); ++b)
-      if (on<R>(j, b)) butterfly<T, L, DIR, Ns, R, PTAB>(v + b * R, tw, j + JS * b);
-  }
-
-  // LDS write of a pass's outputs: component half c (SPLIT) or whole values
-  template <int Ns, int R>
-  __device__ __forceinline__ static void put(const cx<T>* v, unsigned t_in, T* lds, int c) {
-    unsigned t = t_in;
-    asm volatile("" : "+v"(t));
-    const unsigned s = t % (unsigned)TSt, j0 = t / (unsigned)TSt;
-#pragma unroll
-    for (int b = 0; b < rounds<R>(); ++b) {
-      if (!on<R>(j0, b)) continue;
-      const unsigned j = j0 + JS * b, k = j % Ns, base = (j - k) * R + k;
-      const unsigned a0 = LAY::at(s, base);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const unsigned idx = LAY::linear(Ns) ? a0 + r * LAY::delta(Ns) : LAY::at(s, base + r * Ns);
-        if (SPLIT) {
-          lds[idx] = c == 0 ? v[b * R + r].x : v[b * R + r].y;
-        } else {
-          lds[2 * idx] = v[b * R + r].x;
-          lds[2 * idx + 1] = v[b * R + r].y;
-        }
-      }
-    }
-  }
-  template <int R>
-  __device__ __forceinline__ static void get(cx<T>* v, unsigned t_in, const T* lds, int c) {
-    unsigned t = t_in;
-    asm volatile("" : "+v"(t));
-    const unsigned s = t % (unsigned)TSt, j0 = t / (unsigned)TSt;
-#pragma unroll
-    for (int b = 0; b < rounds<R>(); ++b) {
-      if (!on<R>(j0, b)) continue;
-      const unsigned j = j0 + JS * b, a0 = LAY::at(s, j);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const unsigned idx = LAY::linear(L / R) ? a0 + r * LAY::delta(L / R) : LAY::at(s, j + r * (L / R));
-        if (SPLIT) {
-          if (c == 0)
-            v[b * R + r].x = lds[idx];
-          else
-            v[b * R + r].y = lds[idx];
-        } else {
-          v[b * R + r].x = lds[2 * idx];
-          v[b * R + r].y = lds[2 * idx + 1];
-        }
-      }
-    }
-  }
-
-  // passes 1 ... after a first pass (radix R0) whose outputs `put0(c)` writes to LDS
-  template <int Ns, class Put, int R1, int... Rs>
-  __device__ __forceinline__ static void after(Put put_prev, cx<T>* v, unsigned t, T* lds, const cx<T>* tw,
-                                               Plan<R1, Rs...>) {
-#pragma unroll
-    for (int c = 0; c < (SPLIT ? 2 : 1); ++c) {
-      __syncthreads();
-      put_prev(c);
-      __syncthreads();
-      get<R1>(v, t, lds, c);
-    }
-    butterflies<Ns, R1>(v, t, tw);
-    if constexpr (sizeof...(Rs) > 0)
-      after<Ns * R1>([&](int c) { put<Ns, R1>(v, t, lds, c); }, v, t, lds, PTAB ? tw + Ns * R1 : tw, Plan<Rs...>{});
-  }
-};
-
 // The working arrays between the row kernel and the column stage are stored in column
 // blocks of TS modes, [component][k / TS][line][k % TS]: a workgroup's columns are one
 // contiguous run per component, and the TS modes of the consecutive lines that a row

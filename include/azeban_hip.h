@@ -172,9 +172,9 @@ int azb_profile_reset(azb_solver* s);
 
 /* ---- autotuning of the kernel launch shapes --------------------------------
  * Per kernel family (AZB_PROF_*): the column passes take tiles of TS0, TS0/2 or
- * TS0/4 columns (tsdiv 1, 2, 4; TS0 = one 128-byte line), the row kernel P0 or
- * P0/2 line pairs per workgroup (pdiv 1, 2) where it has two shapes (3D N = 64,
- * and FP32 at 3D N = 128; every other row kernel has one).  azb_autotune times
+ * TS0/4 columns (tsdiv 1, 2, 4; TS0 the widest built), the row kernel P0 or
+ * P0/2 line pairs per workgroup (pdiv 1, 2) where it has two shapes (3D FP32 at
+ * N = 64 and 128; every other row kernel has one).  azb_autotune times
  * every candidate on the device with the given state (reps RHS evaluations each,
  * output into the solver's own buffers) and keeps the fastest per family.
  * Results do not depend on the choice.  Synchronising. */
@@ -188,7 +188,9 @@ int azb_get_tuning(const azb_solver* s, int* tsdiv, int* pdiv);
  * agree to round-off, not bit for bit), so solves that must agree bit for bit (a
  * batch and its single solves) use the same plans.  azb_autotune_plans times each
  * plan on the device per family (reps RHS evaluations into the solver's own
- * buffers) and keeps the fastest.  The reference's nearest counterpart is its FFT
+ * buffers) and keeps the fastest; a 2D solver whose column passes are fused with the
+ * k-space update (plan 0 only, faster than the separate passes of any plan) keeps plan 0.
+ * The reference's nearest counterpart is its FFT
  * size choice from a benchmark file (src/azeban/operations/fft.cpp:63-108).
  * Synchronising. */
 int azb_num_plans(const azb_solver* s);
