@@ -1272,7 +1272,9 @@ int azb_autotune_plans(azb_solver* s, const void* u_hat, int reps) {
   if (reps < 1) reps = 3;
   const int n = col_plan_count(s->M);
   if (n == 1) return AZB_OK;
-  if (s->stage.width) {  // the column stage is built for plan 0 and chosen where it beats the separate passes
+  if (s->dim == 2) {
+    // the column stage is built for plan 0; batches that run the separate passes keep it too,
+    // so that they agree with their samples solved alone
     const int zero[AZB_PROF_FAMILIES] = {};
     return azb_set_plans(s, zero);
   }

@@ -188,10 +188,8 @@ int azb_get_tuning(const azb_solver* s, int* tsdiv, int* pdiv);
  * agree to round-off, not bit for bit), so solves that must agree bit for bit (a
  * batch and its single solves) use the same plans.  azb_autotune_plans times each
  * plan on the device per family (reps RHS evaluations into the solver's own
- * buffers) and keeps the fastest; a 2D solver whose column passes are fused with the
- * k-space update (plan 0 only, faster than the separate passes of any plan) keeps plan 0.
- * The reference's nearest counterpart is its FFT
- * size choice from a benchmark file (src/azeban/operations/fft.cpp:63-108).
+ * buffers) and keeps the fastest; 2D solvers keep plan 0, the one whose axis-0 passes are
+ * fused with the k-space update.  The reference's nearest counterpart is its FFT size choice from a benchmark file (src/azeban/operations/fft.cpp:63-108).
  * Synchronising. */
 int azb_num_plans(const azb_solver* s);
 int azb_set_plans(azb_solver* s, const int* plans);
