@@ -483,9 +483,9 @@ __device__ __forceinline__ void butterfly(cx<T>* w, const __attribute__((address
       // chain costs four FMA-class operations and keeps two powers live.
       // Loading every power instead made the 768-point FP64 row kernel 12 %
       // slower (6.39 against 5.72 ms per 512^3 launch), the 2D column stage 11 % at 1024^2; one load per
-      // butterfly (chains of up to 22) measures the same within 1 % and has 1.2-1.4 times the
-      // error of a white-noise RHS (2D 256^2 8.5e-16 against 6.1e-16, 3D 64^3 8.3e-16
-      // against 5.8e-16, both against 80-bit transforms).
+      // butterfly (chains of up to 22) takes the same time (256^3 step 7.60 against 7.57 ms,
+      // 1024^2 204 against 204 us) and has 1.4-1.5 times the error (RHS of a smooth state
+      // against 80-bit transforms: 3D 64^3 4.3e-15 against 2.8e-15, 2D 256^2 2.0e-14 against 1.4e-14).
       const cx<T> w1 = twiddle(k * step);
       cx<T> wr = w1;
       w[1] = cmul_fixed(w[1], w1);
@@ -514,16 +514,14 @@ __device__ __forceinline__ void butterfly(cx<T>* w, const __attribute__((address
 // row of R entries, W^{r k L/(Ns R)} with the transform's direction applied, for
 // r = 1 .. R-1 at row[r-1]) instead of the W_L^e table: one base address per
 // butterfly, constant offsets, 16-byte loads of two FP32 entries.
-// LIVE < TS: the last sequences carry nothing; their slots are neither written nor read.
 template <typename T, int L, int TS, int NT, int DIR, bool SPLIT, int G, int MAPF, int MAPL, bool SWZ = false,
-          int SOFF = 1, unsigned MIDW = 0, int PADE = 0, unsigned MIDH = 0, class LSEL = void, bool PTAB = false, bool CHAIN = sizeof(T) == 8, int LIVE = TS>
+          int SOFF = 1, unsigned MIDW = 0, int PADE = 0, unsigned MIDH = 0, class LSEL = void, bool PTAB = false, bool CHAIN = sizeof(T) == 8>
 struct BlockFFT2 {
   static constexpr int E = TS * L / NT;
   static_assert(TS * L % NT == 0, "TS*L must be a multiple of NT");
   static_assert(MIDW == 0 || (NT == 64 * TS && L == 64 * E), "MAP_WAVE needs one wave per sequence");
   static_assert(MIDH == 0 || (NT == 32 * TS && L == 32 * E), "MAP_HALF needs one half-wave per sequence");
   static_assert((MIDW & MIDH) == 0, "one mapping per pass");
-  static_assert(LIVE == TS || (NT == 32 * TS && G == TS), "idle half-waves");
   using LY = ExLayout<T, L, TS, SWZ, SOFF, PADE>;
   template <int P>
   using XL = typename LaySel<LSEL, P, LY>::type;
@@ -543,13 +541,6 @@ struct BlockFFT2 {
     if (MAP == MAP_WAVE || (MAP == MAP_SEQ1 && L / R == 64 && E == R)) return NT == 64 * TS ? 1 : 0;
     if (MAP == MAP_HALF || (MAP == MAP_SEQ1 && L / R == 32 && E == R)) return NT == 32 * TS ? 2 : 0;
     return 0;
-  }
-  // whether butterfly b of this thread belongs to a sequence that carries values
-  template <int MAP>
-  __device__ __forceinline__ static bool live(unsigned t, int b) {
-    if (LIVE == TS) return true;
-    if (MAP == MAP_SEQ) return b % G < LIVE;
-    return t < 32u * LIVE;  // half-wave per sequence
   }
   // Between the write and the read phases of an exchange, and before the writes
   // (earlier reads of the same words): a workgroup barrier, or, when both mappings
@@ -604,7 +595,6 @@ struct BlockFFT2 {
       exchange_sync<local>();
 #pragma unroll
       for (int b = 0; b < E / R; ++b) {
-        if (!live<MAPW>(t, b)) continue;
         unsigned s, j;
         bmap<MAPW, TS, NT, L, R, G>(t, b, s, j);
         const unsigned k = j % Ns;
@@ -624,7 +614,6 @@ struct BlockFFT2 {
       exchange_sync<local>();
 #pragma unroll
       for (int b = 0; b < E / Rn; ++b) {
-        if (!live<MAPR>(t, b)) continue;
         unsigned s, j;
         bmap<MAPR, TS, NT, L, Rn, G>(t, b, s, j);
         const unsigned a0 = XLY::at(s, j);
@@ -662,78 +651,6 @@ struct BlockFFT2 {
   __device__ __forceinline__ static void run(cx<T>* v, int t, T* lds, const cx<T>* tw, Plan<Rs...> p) {
     static_assert(plan_prod<Rs...>() == L, "plan must multiply to L");
     passes<0, PlanAt<Rs...>::count, 1, Rs...>(v, t, lds, tw, p);
-  }
-
-  // run() for a last radix RL that does not divide a thread's E values (RL > E): the first
-  // TS L / RL threads take one last-pass butterfly each (MAP_SEQ1), the others none.  The
-  // array v holds RL values.
-  template <int P, int NP, int Ns, int R, int RL>
-  __device__ __forceinline__ static void wide_passes(cx<T>* v, int t, T* lds, const cx<T>* tw, Plan<R, RL>) {
-    static_assert(!PTAB && TS * L / RL <= NT && MAPL == MAP_SEQ1, "one last-pass butterfly per thread");
-    constexpr int MAPW = map_of<P, NP>();
-    using XLY = XL<P>;
-    butterflies<MAPW, Ns, R>(v, t, tw);
-    unsigned tt = t;
-    asm volatile("" : "+v"(tt));
-    __builtin_assume(tt < (unsigned)NT);
-    const bool mine = tt < (unsigned)(TS * L / RL);
-    const unsigned s1 = tt / (unsigned)(L / RL), j1 = tt % (unsigned)(L / RL);
-    cx<T> x[RL];
-#pragma unroll
-    for (int c = 0; c < (SPLIT ? 2 : 1); ++c) {
-      __syncthreads();
-#pragma unroll
-      for (int b = 0; b < E / R; ++b) {
-        unsigned s, j;
-        bmap<MAPW, TS, NT, L, R, G>(tt, b, s, j);
-        const unsigned k = j % Ns, base = (j - k) * R + k, a0 = XLY::at(s, base);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const unsigned idx = XLY::linear(Ns) ? a0 + r * XLY::delta(Ns) : XLY::at(s, base + r * Ns);
-          if (SPLIT) {
-            lds[idx] = c == 0 ? v[b * R + r].x : v[b * R + r].y;
-          } else {
-            lds[2 * idx] = v[b * R + r].x;
-            lds[2 * idx + 1] = v[b * R + r].y;
-          }
-        }
-      }
-      __syncthreads();
-      if (mine) {
-        const unsigned a0 = XLY::at(s1, j1);
-#pragma unroll
-        for (int r = 0; r < RL; ++r) {
-          const unsigned idx = XLY::linear(L / RL) ? a0 + r * XLY::delta(L / RL) : XLY::at(s1, j1 + r * (L / RL));
-          if (SPLIT) {
-            if (c == 0)
-              x[r].x = lds[idx];
-            else
-              x[r].y = lds[idx];
-          } else {
-            x[r].x = lds[2 * idx];
-            x[r].y = lds[2 * idx + 1];
-          }
-        }
-      }
-    }
-    if (mine) butterfly<T, L, DIR, Ns * R, RL, false, CHAIN>(x, (twptr)tw, j1);
-#pragma unroll
-    for (int r = 0; r < RL; ++r) v[r] = x[r];
-  }
-  template <int P, int NP, int Ns, int R, int Rn, int Rm, int... Rs>
-  __device__ __forceinline__ static void wide_passes(cx<T>* v, int t, T* lds, const cx<T>* tw,
-                                                     Plan<R, Rn, Rm, Rs...>) {
-    butterflies<map_of<P, NP>(), Ns, R>(v, t, tw);
-    exchange<map_of<P, NP>(), map_of<P + 1, NP>(), Ns, R, Rn, XL<P>>(v, t, lds);
-    wide_passes<P + 1, NP, Ns * R>(v, t, lds, tw, Plan<Rn, Rm, Rs...>{});
-  }
-  template <int... Rs>
-  __device__ __forceinline__ static void run_wide(cx<T>* v, int t, T* lds, const cx<T>* tw, Plan<Rs...> p) {
-    static_assert(plan_prod<Rs...>() == L, "plan must multiply to L");
-    if constexpr (E % last_radix(Plan<Rs...>{}) == 0)
-      run(v, t, lds, tw, p);
-    else
-      wide_passes<0, PlanAt<Rs...>::count, 1>(v, t, lds, tw, p);
   }
 
   // run() after load_dft(): the first pass's butterflies are already applied

@@ -175,24 +175,21 @@ __global__ void stage_modes_kernel(double2* modes, int N, int nh, double eps, do
 
 // The lines below were placed by timing whole steps (device loop, Fourier states of a
 // shear layer; us per step against the separate passes of the same size, FP64 / FP32).
-// A CU holds one workgroup of 12 waves (134-168 registers), so what counts is the number
+// A CU holds one workgroup of 12 waves (148-168 registers), so what counts is the number
 // of rounds of 256 workgroups and how full the last one is.
-//   N = 64, 128  : width 4, split 2 whatever the batch (N = 64: 54 / 51 against 81 / 101;
-//                  N = 128 x 33: 94 / 84 against 128 / 149)
-//   N = 256      : width 2, split 2 until the wider tiles fill the chip (one sample 72 / 70
-//                  against 107 / 129), then width 4 (x 21: 166 / 140 against 227 / 215; width 2
-//                  190 in FP64)
-//   N = 512      : one sample width 2, split 2 (92 / 84 against 124 / 136); batches whole
-//                  lines (width 8) unless width 4, split 2 needs less than 1.7 (FP32: 1.9) times
-//                  the rounds (x 13: 415 / 320 against 458 / 361, width 4 444 in FP64; x 64 FP64:
-//                  1736 against 1935, width 4 1865; x 8 FP64: 315 at width 4 against 326 at
-//                  width 8).  FP32 batches whose last round is less than a fifth short stay
-//                  ahead of the separate passes (x 64: 1516 against 1519), the others do not
-//                  (x 8: 281 against 265, x 24: 653 against 624)
-//   N = 1024     : one sample width 4 (177 / 162 against 210 / 194).  FP64 batches too once
-//                  there are fewer rounds than samples (x 8, five rounds: 1052 against 1198);
-//                  two need two rounds for 258 workgroups (349 / 320 against 329 / 298), so
-//                  those and FP32 batches keep the separate passes
+//   N = 64, 128  : width 4, split 2 whatever the batch (N = 64: 57 / 51 against 86 / 101;
+//                  N = 128 x 33: 115 / 84 against 160 / 149)
+//   N = 256      : width 2, split 2 until the wider tiles fill the chip (one sample 78 / 70
+//                  against 119 / 129), then width 4 (x 21: 204 / 140 against 274 / 215)
+//   N = 512      : one sample width 2, split 2 (104 / 84 against 137 / 136); batches whole
+//                  lines (width 8) unless width 4, split 2 needs less than 1.9 times the
+//                  rounds (x 13: 518 / 320 against 546 / 361; x 8 FP64: 360 at width 4
+//                  against 404 at width 8).  FP32 batches whose last round is less than
+//                  a fifth short stay ahead of the separate passes (x 64: 1516 against
+//                  1519), the others do not (x 8: 281 against 265, x 24: 653 against 624)
+//   N = 1024     : one sample width 4 (207 / 162 against 234 / 194); two need two rounds for
+//                  258 workgroups (415 / 320 against 390 / 298), so batches keep the
+//                  separate passes
 StageShape stage_shape(int tbytes, int L, long nsamples) {
   const long nh = L / 3 + 1;
   auto wgs = [&](int w) { return (nh + w - 1) / w * nsamples; };
@@ -202,13 +199,12 @@ StageShape stage_shape(int tbytes, int L, long nsamples) {
     case 384: return wgs(4) <= 256 ? StageShape{2, 2} : StageShape{4, 1};
     case 768: {
       if (nsamples == 1) return {2, 2};
-      const bool wide = (tbytes == 8 ? 1.7 : 1.9) * rounds(8) <= rounds(4);
+      const bool wide = 1.9 * rounds(8) <= rounds(4);
       if (tbytes == 8) return wide ? StageShape{8, 1} : StageShape{4, 2};
       if (rounds(8) == 1) return wide ? StageShape{8, 1} : StageShape{4, 2};
       return wgs(8) >= 0.8 * 256 * rounds(8) ? StageShape{8, 1} : StageShape{0, 0};
     }
-    case 1536:
-      return nsamples == 1 || (tbytes == 8 && rounds(4) < nsamples) ? StageShape{4, 1} : StageShape{0, 0};
+    case 1536: return nsamples == 1 ? StageShape{4, 1} : StageShape{0, 0};
     default: return {0, 0};
   }
 }

@@ -292,38 +292,23 @@ __device__ __forceinline__ double sv_eval(double k, double eps, double s2, doubl
   return -eps * kp * qk;
 }
 
-// Products the RHS transforms back.  FP64: the last diagonal one is taken off the others
-// (2D: B11 - B22, B12; 3D: B11 - B33, B21, B22 - B33, B31, B32), which changes B by a
-// multiple of the identity, its divergence by a gradient, and so nothing after the Leray
-// projection, for every mode.  A sixth (2D: a third) of the forward passes' and the k-space
-// kernel's traffic and transforms goes: a step at 512^3 56.7 -> 52.1 ms, 256^3 7.4 -> 6.8,
-// 64^3 215 -> 191 us, eight 2D steps at 1024^2 1.64 -> 1.36 ms, an ensemble 6.8 -> 5.5 ms.
-// RHS error against 80-bit transforms, together with the shorter twiddle chains, before and
-// after: 3D Brownian 128^3 5.0e-15 / 4.0e-15, 64^3 3.0e-15 / 2.2e-15; 2D white noise 256^2
-// 8.6e-16 / 6.1e-16, shear layer 1024^2 2.3e-13 / 1.9e-13, 512^2 7.7e-14 / 7.6e-14.  A state
-// u = (g(y), f(x)) exactly, where every line's B11 is the same and its noise cancelled, loses
-// that: shear layer 64^2 7.5e-15 / 8.3e-15, 256^2 3.3e-14 / 3.8e-14 (its first RHS only).
-// FP32: all products, since there the changed rounding (1e-7) would show in FP64 states.
-template <typename T, int DIM>
-constexpr int products() { return 3 * (DIM - 1) - (sizeof(T) == 8 ? 1 : 0); }
-
 // One mode's wavevector, |k|^2 and Leray projector 1 - k k^T / |k|^2 (symmetric:
 // P11, P12, P22 in 2D; P11, P21, P22, P31, P32, P33 in 3D).
 constexpr double kTwoPi = 2.0 * 3.14159265358979323846;
 template <int DIM>
 struct ModeGeom {
-  double k[3], P[6], absk2, inv;  // inv = 1 / |k|^2
+  double k[3], P[6], absk2;
   // 2D: signed mode number i of axis 0, kk of the last axis, inv = 1 / |k|^2 from the
   // caller's table, or computed here
-  __device__ __forceinline__ void set2(int i, int kk, double inv_, bool have_inv) {
+  __device__ __forceinline__ void set2(int i, int kk, double inv, bool have_inv) {
     const double k1 = kTwoPi * i, k2 = kTwoPi * kk;
     absk2 = k1 * k1 + k2 * k2;
-    inv = have_inv ? inv_ : 1.0 / absk2;
+    if (!have_inv) inv = 1.0 / absk2;
     const double k11 = k1 * k1 * inv, k12 = k1 * k2 * inv, k22 = k2 * k2 * inv;
     k[0] = k1; k[1] = k2;
     P[0] = 1.0 - k11; P[1] = 0.0 - k12; P[2] = 1.0 - k22;
   }
-  __device__ __forceinline__ ModeGeom(int i, int kk, double inv_) { set2(i, kk, inv_, true); }
+  __device__ __forceinline__ ModeGeom(int i, int kk, double inv) { set2(i, kk, inv, true); }
   // signed mode numbers i, j of the full axes (2D: i only), kk of the last
   __device__ __forceinline__ ModeGeom(int i, int j, int kk) {
     if (DIM == 2) {
@@ -332,7 +317,7 @@ struct ModeGeom {
     }
     const double k1 = kTwoPi * i, k2 = kTwoPi * j, k3 = kTwoPi * kk;
     absk2 = k1 * k1 + k2 * k2 + k3 * k3;
-    inv = 1.0 / absk2;
+    const double inv = 1.0 / absk2;
     const double k11 = k1 * k1 * inv, k12 = k1 * k2 * inv, k13 = k1 * k3 * inv;
     const double k22 = k2 * k2 * inv, k23 = k2 * k3 * inv, k33 = k3 * k3 * inv;
     k[0] = k1; k[1] = k2; k[2] = k3;
@@ -344,19 +329,16 @@ struct ModeGeom {
 // b = k . B for one half (real or imaginary parts) of the products B_m at a mode: ik.B_hat
 // maps Re B to the imaginary part of b and -Im B to its real part, so the two halves never
 // meet and a caller may hold one at a time.
-// NM products; the last diagonal one may be left out (see products()).  In 2D only one
-// number of b then matters, its part along (k2, -k1), which is all that the Leray
-// projection keeps: b[0] = k2 b1 - k1 b2 = k1 k2 B_0 + (k2^2 - k1^2) B_1.
-template <int DIM, int NM>
-constexpr int dot_values() { return DIM == 2 && NM == 2 ? 1 : DIM; }
-template <int DIM, int NM>
+// Every product is transformed.  Taking the last diagonal one off the others (a gradient, which
+// the projection removes) saves a sixth of the forward work, a third in 2D (512^3 step 59.5 ->
+// 53.6 ms), but mixes the squares' roundings: eps u3^2 then enters equations that u3^2 itself
+// has no effect on.  In-plane du/dt of a 64^3 flow invariant along z with u3 = 100 |u1, u2|:
+// 2.6e-11 instead of 3.3e-15 off 80-bit transforms, a separable 2D shear layer's (ratio 1000) 2.8e-13
+// instead of 2.0e-15, and taking off the smallest component's square instead helps only
+// the first (u = (U(y), 1e-3 f(x), 7e-4 f(-x)): 8.2e-13 instead of 3.5e-15).
+template <int DIM>
 __device__ __forceinline__ void kspace_dot(const ModeGeom<DIM>& g, const double* B, double* b) {
-  constexpr bool ALL = NM == 3 * (DIM - 1);
-  if constexpr (DIM == 2 && !ALL) {
-    const double k1 = g.k[0], k2 = g.k[1];
-    const double x = (k1 * k2) * B[0], y = ((k2 - k1) * (k2 + k1)) * B[1];
-    b[0] = x + y;
-  } else if constexpr (DIM == 2) {
+  if (DIM == 2) {
     const double t1 = g.k[0] * B[0], t2 = g.k[1] * B[1];
     const double t3 = g.k[0] * B[1], t4 = g.k[1] * B[2];
     b[0] = t1 + t2;
@@ -371,25 +353,16 @@ __device__ __forceinline__ void kspace_dot(const ModeGeom<DIM>& g, const double*
       b[1] = x + y + z;
     }
     {
-      const double x = g.k[0] * B[3], y = g.k[1] * B[4];
-      if constexpr (ALL) {
-        const double z = g.k[2] * B[5];
-        b[2] = x + y + z;
-      } else {
-        b[2] = x + y;
-      }
+      const double x = g.k[0] * B[3], y = g.k[1] * B[4], z = g.k[2] * B[5];
+      b[2] = x + y + z;
     }
   }
 }
 
-// L = P b, the Leray projection of one half, from kspace_dot's values
-template <int DIM, int NM>
+// L = P b, the Leray projection of one half
+template <int DIM>
 __device__ __forceinline__ void kspace_project(const ModeGeom<DIM>& g, const double* b, double* L) {
-  if constexpr (DIM == 2 && NM == 2) {
-    const double w = b[0] * g.inv;
-    L[0] = g.k[1] * w;
-    L[1] = -g.k[0] * w;
-  } else if constexpr (DIM == 2) {
+  if (DIM == 2) {
     L[0] = g.P[0] * b[0] + g.P[1] * b[1];
     L[1] = g.P[1] * b[0] + g.P[2] * b[1];
   } else {
@@ -414,7 +387,7 @@ __device__ __forceinline__ double stage_value(int mode, double absk2, double L, 
 template <typename T, int DIM, int MODE>
 __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
   // grid.y = sample; samples are stacked with strides DIM*nmodes (state) and
-  // NM*bstride (B_hat)
+  // 3(DIM-1)*bstride (B_hat)
   const long sample = blockIdx.y;
   DevState* st = a.st + sample;
   if (st->done) return;
@@ -443,8 +416,7 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= a.nmodes) return;
   const int N = a.n, NH = a.nh;
-  constexpr int NM = products<T, DIM>();
-  const cx<T>* bh = (const cx<T>*)a.bh + sample * NM * a.bstride;
+  const cx<T>* bh = (const cx<T>*)a.bh + sample * (3 * (DIM - 1)) * a.bstride;
   // 32-bit index arithmetic: the supported grids have fewer than 2^27 modes per component
   const unsigned ui = (unsigned)idx;
   const int kk = (int)(ui % (unsigned)NH);
@@ -453,6 +425,7 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
   const int j = DIM == 3 ? (int)(rest % (unsigned)N) : 0;
   const int i = DIM == 3 ? (int)(rest / (unsigned)N) : (int)rest;
   const ModeGeom<DIM> g(i >= N / 2 + 1 ? i - N : i, j >= N / 2 + 1 ? j - N : j, kk);
+  constexpr int NM = 3 * (DIM - 1);
   double Br[NM], Bi[NM], b[DIM], Lr[DIM], Li[DIM];
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
@@ -460,10 +433,10 @@ __global__ __launch_bounds__(256) void kspace_kernel(KArgs a) {
     Br[m] = (double)z.x;
     Bi[m] = -(double)z.y;
   }
-  kspace_dot<DIM, NM>(g, Bi, b);
-  kspace_project<DIM, NM>(g, b, Lr);
-  kspace_dot<DIM, NM>(g, Br, b);
-  kspace_project<DIM, NM>(g, b, Li);
+  kspace_dot<DIM>(g, Bi, b);
+  kspace_project<DIM>(g, b, Lr);
+  kspace_dot<DIM>(g, Br, b);
+  kspace_project<DIM>(g, b, Li);
   const double nu = sv_eval(sqrt(g.absk2), a.eps, a.s2, a.k0);
 #pragma unroll
   for (int c = 0; c < DIM; ++c) {
@@ -869,10 +842,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // ---------------------------------------------------------------------------
 // 3D FP64 row kernel at L = 768 with one forward round.  The inverse is the row-4
 // kernel's (three packed sequences of one line pair, 12 values per thread, plan
-// 12.4.4.4).  All five products B_m (packed line a + i line b, see products()) are formed
-// at once from the inverse output, so the inverse values need not stay in registers for a
-// second round, and one forward transform in a layout for six sequences (24 values per
-// thread, plan 4.8.24, two exchanges; the sixth half-wave idles) replaces the row-4 kernel's two rounds of three
+// 12.4.4.4).  All six products B_m (packed line a + i line b) are formed at once
+// from the inverse output, so the inverse values need not stay in registers for a
+// second round, and one forward transform of six sequences (24 values per thread,
+// plan 4.8.24, two exchanges) replaces the row-4 kernel's two rounds of three
 // (three exchanges each).  The forward exchanges go in two halves (real,
 // imaginary: 8-byte slots, pad period 32) so the exchange buffer keeps the size
 // of the inverse's.  The radix-24 last pass keeps butterfly j of sequence m in
@@ -922,11 +895,8 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // radix-24 pass (half-wave per sequence too) needs none either
   using FI = BlockFFT2<T, L, 3, NT, +1, false, 3, MAP_SEQ1, MAP_SEQ, true, C::SOFFI, 0b0110u, 0, 0u,
                        typename C::InvLay>;
-  // five products in a layout for six sequences: the sixth half-wave stays out of the
-  // exchanges and stores nothing
-  constexpr int NM = products<T, 3>();
   using FF = BlockFFT2<T, L, 6, NT, -1, true, 6, MAP_SEQ, MAP_SEQ1, true, C::SOFFF, 0u, 32, 0b010u,
-                       typename C::FwdLay, false, true, NM>;
+                       typename C::FwdLay>;
   static_assert(FI::E == EI && FF::E == EF, "thread layout");
   static_assert(FI::lds_words <= C::XWORDS && FF::lds_words <= C::XWORDS, "exchange size");
   __shared__ T X[C::XWORDS];
@@ -961,29 +931,27 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   asm volatile("" : "+v"(lmax));
 
   // products at this thread's 4 positions: w[m*4 + r] = B_m (line a) + i B_m (line b),
-  // m = 0..4: B11 - B33, B21, B22 - B33, B31, B32
+  // m = 0..5: B11, B21, B22, B31, B32, B33
   cx<T> w[EF];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const cx<T> p0 = u[r], p1 = u[4 + r], p2 = u[8 + r];
     const T a1 = nrm * p0.x, a2 = nrm * p0.y, a3 = nrm * p1.x;
     const T b1 = nrm * p2.x, b2 = nrm * p2.y, b3 = nrm * p1.y;
-    const T a33 = a3 * a3, b33 = b3 * b3;
-    w[0 * 4 + r] = mk(a1 * a1 - a33, b1 * b1 - b33);
+    w[0 * 4 + r] = mk(a1 * a1, b1 * b1);
     w[1 * 4 + r] = mk(a2 * a1, b2 * b1);
-    w[2 * 4 + r] = mk(a2 * a2 - a33, b2 * b2 - b33);
+    w[2 * 4 + r] = mk(a2 * a2, b2 * b2);
     w[3 * 4 + r] = mk(a3 * a1, b3 * b1);
     w[4 * 4 + r] = mk(a3 * a2, b3 * b2);
-    w[5 * 4 + r] = mk(T(0), T(0));
+    w[5 * 4 + r] = mk(a3 * a3, b3 * b3);
   }
   FF::run(w, t, X, tw, Plan<4, 8, 24>{});
   {
     unsigned tt = t;
     asm volatile("" : "+v"(tt));
     const unsigned m = tt / NBF, j = tt % NBF;
-    if (m < (unsigned)NM)
-      row_separate_store<T, NBF, 24>(w, tt & 63, j, (vec2_t<T>*)(out + ((long)m * a.nlines + la) * a.ls),
-                                     (vec2_t<T>*)(out + ((long)m * a.nlines + lb) * a.ls));
+    row_separate_store<T, NBF, 24>(w, tt & 63, j, (vec2_t<T>*)(out + ((long)m * a.nlines + la) * a.ls),
+                                   (vec2_t<T>*)(out + ((long)m * a.nlines + lb) * a.ls));
   }
 
   lmax = wave_max<T>(lmax);
@@ -1004,9 +972,9 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // runs on the first 2P * L/12 = 128 threads, one butterfly each, the later passes
 // on all threads with 8 values each; the last pass (radix 4, MAP_SEQ) leaves u1, u2
 // of both lines of a pair at the same four positions in one thread.  Products
-// (FP64: B11 - B22, B12; FP32: B11, B12, B22) packed (line a) + i (line b) feed the forward
-// transform (2P or 3P sequences, 8 or 12 values per thread) at those positions; its radix-12
-// last pass, in FP64 on 128 threads (BlockFFT2::run_wide), separates the two half spectra over lane permutes as in the 3D kernel.
+// (B11, B12, B22) packed (line a) + i (line b) feed the forward transform (3P
+// sequences, 12 values per thread) at those positions; its radix-12 last pass
+// separates the two half spectra over lane permutes as in the 3D kernel.
 // ---------------------------------------------------------------------------
 template <int L>
 struct Row2Plan;
@@ -1018,8 +986,7 @@ struct Row2Cfg {
   static_assert(L <= 192, "L = 384, 768 and 1536 have kernels of their own (euler_row2p_kernel, euler_row2w_kernel)");
   static constexpr int P = 768 / L;
   static constexpr int NT = P * L / 4;
-  static constexpr int NM = products<T, 2>();
-  static constexpr int TSI = 2 * P, TSF = NM * P;
+  static constexpr int TSI = 2 * P, TSF = 3 * P;
   static constexpr int NB = L / 12;
   static constexpr int SOFF = 11;
   static constexpr int XI = 2 * ExLayout<T, L, TSI, true, SOFF>::elems;
@@ -1033,10 +1000,10 @@ __global__ __launch_bounds__((Row2Cfg<T, L>::NT)) void euler_row2_kernel(RowArgs
   using PL = Row2Plan<L>;
   constexpr int NT = C::NT, P = C::P, NB = C::NB, TSI = C::TSI, TSF = C::TSF;
   using FI = BlockFFT2<T, L, TSI, NT, +1, false, 2, MAP_STD, MAP_SEQ, true, C::SOFF>;
-  constexpr int MAPL = MAP_SEQ1, NM = C::NM;
-  using FF = BlockFFT2<T, L, TSF, NT, -1, false, NM, MAP_SEQ, MAPL, true, C::SOFF>;
-  using LY = ExLayout<T, L, TSI, true, C::SOFF>;
-  static_assert(FI::E == 8 && FF::E == 4 * NM, "thread layout");
+  constexpr int MAPL = MAP_SEQ1;
+  using FF = BlockFFT2<T, L, TSF, NT, -1, false, 3, MAP_SEQ, MAPL, true, C::SOFF>;
+  using LY = ExLayout<T, L, TSF, true, C::SOFF>;
+  static_assert(FI::E == 8 && FF::E == 12, "thread layout");
   static_assert(64 % NB == 0 && TSI * NB % 64 == 0, "whole waves in the radix-12 passes");
   static_assert(first_radix(typename PL::Inv{}) == 12 && last_radix(typename PL::Inv{}) == 4 &&
                     first_radix(typename PL::Fwd{}) == 4 && last_radix(typename PL::Fwd{}) == 12,
@@ -1086,21 +1053,18 @@ __global__ __launch_bounds__((Row2Cfg<T, L>::NT)) void euler_row2_kernel(RowArgs
     const cx<T> pa = v[r], pb = v[4 + r];
     lm = fmax(lm, fmax(fmax(fabs(pa.x), fabs(pa.y)), fmax(fabs(pb.x), fabs(pb.y))));
     const T a1 = nrm * pa.x, a2 = nrm * pa.y, b1 = nrm * pb.x, b2 = nrm * pb.y;
+    w[r] = mk(a1 * a1, b1 * b1);      // B11
     w[4 + r] = mk(a1 * a2, b1 * b2);  // B12
-    if constexpr (NM == 2) {
-      w[r] = mk(a1 * a1 - a2 * a2, b1 * b1 - b2 * b2);  // B11 - B22
-    } else {
-      w[r] = mk(a1 * a1, b1 * b1);      // B11
-      w[8 + r] = mk(a2 * a2, b2 * b2);  // B22
-    }
+    w[8 + r] = mk(a2 * a2, b2 * b2);  // B22
   }
   double lmax = (double)lm;
-  FF::run_wide(w, t, X, tw, typename PL::Fwd{});
-  if (t < TSF * NB) {
+  FF::run(w, t, X, tw, typename PL::Fwd{});
+  {
     unsigned tt = t;
     asm volatile("" : "+v"(tt));
-    const unsigned s = tt / NB, j = tt % NB;
-    const unsigned pair = s / NM, m = s % NM;
+    unsigned s, j;
+    bmap<MAPL, TSF, NT, L, 12, 3>(tt, 0, s, j);
+    const unsigned pair = s / 3, m = s % 3;
     const long la = line0 + 2 * pair, lb = la + 1;
     row_separate_store<T, NB, 12>(w, tt & 63, j, (vec2_t<T>*)(out + m * cs + la * a.ls),
                               (vec2_t<T>*)(out + m * cs + lb * a.ls), cols);
@@ -1123,10 +1087,8 @@ __global__ __launch_bounds__((Row2Cfg<T, L>::NT)) void euler_row2_kernel(RowArgs
 // first pass from HBM on 128 threads (butterfly j of sequence s, NB = 64), written
 // to LDS, then two radix-8 passes on all 192 threads with 16 values each; the last
 // leaves u1 + i u2 of both lines at the same eight positions t + 192 r in thread t.
-// Forward (plan 8.8.24).  FP64: two sequences (B11 - B22, B12 packed line a + i line b), 16
-// values per thread, exchanges in real/imaginary halves, the radix-24 pass on two waves
-// (BlockFFT2::run_wide).  FP32: three sequences (B11, B12, B22), 24
-// values per thread: the radix-8 middle pass
+// Forward (plan 8.8.24, three sequences B11, B12, B22 packed line a + i line b, 24
+// values per thread, exchanges in real/imaginary halves): the radix-8 middle pass
 // keeps each sequence in its own wave, so the exchange into the radix-24 pass (one
 // sequence per wave, butterfly j in lane j) needs no workgroup barrier, and the
 // separation of each packed spectrum stays within a wave.  Two exchanges per
@@ -1151,10 +1113,9 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void e
   constexpr int L = C::L, NT = C::NT, NB = C::NB;
   // forward exchange halves in FP64 (8-byte slots) keep the buffer at the inverse's
   using FI = BlockFFT2<T, L, 2, NT, +1, false, 2, MAP_STD, MAP_SEQ, true, C::SOFF>;
-  constexpr int NM = products<T, 2>();
-  using FF = BlockFFT2<T, L, NM, NT, -1, sizeof(T) == 8, NM, MAP_SEQ, MAP_SEQ1, true, C::SOFF, NM == 3 ? 0b010u : 0u>;
+  using FF = BlockFFT2<T, L, 3, NT, -1, sizeof(T) == 8, 3, MAP_SEQ, MAP_SEQ1, true, C::SOFF, 0b010u>;
   using LY = ExLayout<T, L, 2, true, C::SOFF>;
-  static_assert(FI::E == 16 && FF::E == 8 * NM, "thread layout");
+  static_assert(FI::E == 16 && FF::E == 24, "thread layout");
   constexpr int XWORDS = FI::lds_words > FF::lds_words ? FI::lds_words : FF::lds_words;
   __shared__ T X[XWORDS];
   __shared__ double red[NT / 64];
@@ -1201,18 +1162,14 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void e
     const cx<T> pa = v[r], pb = v[8 + r];
     lm = fmax(lm, fmax(fmax(fabs(pa.x), fabs(pa.y)), fmax(fabs(pb.x), fabs(pb.y))));
     const T a1 = nrm * pa.x, a2 = nrm * pa.y, b1 = nrm * pb.x, b2 = nrm * pb.y;
-    w[8 + r] = mk(a1 * a2, b1 * b2);  // B12
-    if constexpr (NM == 2) {
-      w[r] = mk(a1 * a1 - a2 * a2, b1 * b1 - b2 * b2);  // B11 - B22
-    } else {
-      w[r] = mk(a1 * a1, b1 * b1);       // B11
-      w[16 + r] = mk(a2 * a2, b2 * b2);  // B22
-    }
+    w[r] = mk(a1 * a1, b1 * b1);       // B11
+    w[8 + r] = mk(a1 * a2, b1 * b2);   // B12
+    w[16 + r] = mk(a2 * a2, b2 * b2);  // B22
   }
   double lmax = (double)lm;
   asm volatile("" : "+v"(lmax));
-  FF::run_wide(w, t, X, tw, typename C::PF{});
-  if (t < NM * NB) {
+  FF::run(w, t, X, tw, typename C::PF{});
+  {
     unsigned tt = t;
     asm volatile("" : "+v"(tt));
     const unsigned m = tt / NB, j = tt % NB;
@@ -1233,12 +1190,11 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void e
 
 // ---------------------------------------------------------------------------
 // 2D row kernel at L = 768 and 384 (N = 512, 256) with P = 1536/L line pairs per
-// 192-thread workgroup, plans 4.8.24 / 4.4.24, every exchange in real/imaginary halves.
-// FP64: 2P sequences (B11 - B22, B12 of each pair, packed line a + i line b), 16 values per
-// thread, the radix-24 pass on 128 threads (BlockFFT2::run_wide); at L = 768
-// euler_row6_kernel's swizzled second exchange.  FP32: 3P sequences (B11, B12, B22), 24
-// values per thread; at L = 768 as euler_row8_kernel, the radix-8 pass in half-waves,
-// per-pass twiddle tables.  Inverse (plans 24.8.4 / 24.4.4):
+// 192-thread workgroup and the 3D kernels' forward: 3P sequences (B11, B12, B22 of
+// each pair, packed line a + i line b), 24 values per thread, plans 4.8.24 / 4.4.24
+// (at L = 768 the radix-8 pass in half-waves; FP64 as euler_row6_kernel, swizzled
+// second exchange; FP32 as euler_row8_kernel, per-pass twiddle tables; every
+// exchange in real/imaginary halves).  Inverse (plans 24.8.4 / 24.4.4):
 // the radix-24 first pass from HBM on 128 threads (2P sequences u1 + i u2 of lines
 // 0..2P-1, butterfly j in lane j of an L/24-lane group), written to LDS, then 16
 // values per thread on all 192 threads; the radix-4 last pass leaves four
@@ -1268,18 +1224,15 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   // per-pass twiddle tables: FP32 at L = 768 (the 3D FP32 row kernel's, same plans)
   constexpr bool PT = F32 && L == 768;
   using FI = BlockFFT2<T, L, 2 * P, NT, +1, SPI, 4, MAP_STD, MAP_SEQ, true, C::SOFFI, 0u, 0, 0u, void, PT>;
-  constexpr int NM = products<T, 2>();
-  // the radix-8 pass in half-waves, the exchange after it without a barrier (FP32, whose
-  // six sequences of 24 values fill them)
   using FF768 = std::conditional_t<
       F32, BlockFFT2<T, L, 6, NT, -1, true, 6, MAP_SEQ, MAP_SEQ1, true, 5, 0u, 0, 0b010u, void, true>,
-      BlockFFT2<T, L, NM * P, NT, -1, true, 2 * NM, MAP_SEQ, MAP_SEQ1, true, Row6Cfg::SOFFF, 0u, 32, 0u,
+      BlockFFT2<T, L, 6, NT, -1, true, 6, MAP_SEQ, MAP_SEQ1, true, Row6Cfg::SOFFF, 0u, 32, 0b010u,
                 typename Row6Cfg::FwdLay>>;
-  using FF384 = BlockFFT2<T, L, NM * P, NT, -1, true, 2 * NM, MAP_SEQ, MAP_SEQ1, true, 5, 0u, F32 ? 0 : 32>;
+  using FF384 = BlockFFT2<T, L, 3 * P, NT, -1, true, 6, MAP_SEQ, MAP_SEQ1, true, 5, 0u, F32 ? 0 : 32>;
   using FF = std::conditional_t<L == 768, FF768, FF384>;
   using LY = ExLayout<T, L, 2 * P, true, C::SOFFI>;
   static_assert(std::is_same_v<LY, typename FI::template XL<0>>, "first-pass layout");
-  static_assert(FI::E == 16 && FF::E == 8 * NM, "thread layout");
+  static_assert(FI::E == 16 && FF::E == 24, "thread layout");
   constexpr int XWORDS = FI::lds_words > FF::lds_words ? FI::lds_words : FF::lds_words;
   static_assert(L == 768 || 4 * (XWORDS * (int)sizeof(T) + 3 * 8) <= 163840, "four workgroups per CU");
   __shared__ T X[XWORDS];
@@ -1362,7 +1315,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
 
   // v[g*4 + r]: u1 + i u2 of line 4 (t / (L/4)) + g (g = 0..3) at positions
   // t % (L/4) + (L/4) r; products of the thread's pair p (lines 2p, 2p + 1 of the
-  // four) into its sequences NM p + m, m = B11, B12, B22 (see products())
+  // four) into its sequences 3p + m, m = B11, B12, B22
   T lm = T(0);
   cx<T> w[24];
 #pragma unroll
@@ -1372,24 +1325,19 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
       const cx<T> pa = v[(2 * p) * 4 + r], pb = v[(2 * p + 1) * 4 + r];
       lm = fmax(lm, fmax(fmax(fabs(pa.x), fabs(pa.y)), fmax(fabs(pb.x), fabs(pb.y))));
       const T a1 = nrm * pa.x, a2 = nrm * pa.y, b1 = nrm * pb.x, b2 = nrm * pb.y;
-      cx<T>* x = w + (NM * p) * 4 + r;
-      x[4] = mk(a1 * a2, b1 * b2);  // B12
-      if constexpr (NM == 2) {
-        x[0] = mk(a1 * a1 - a2 * a2, b1 * b1 - b2 * b2);  // B11 - B22
-      } else {
-        x[0] = mk(a1 * a1, b1 * b1);  // B11
-        x[8] = mk(a2 * a2, b2 * b2);  // B22
-      }
+      w[(3 * p) * 4 + r] = mk(a1 * a1, b1 * b1);      // B11
+      w[(3 * p + 1) * 4 + r] = mk(a1 * a2, b1 * b2);  // B12
+      w[(3 * p + 2) * 4 + r] = mk(a2 * a2, b2 * b2);  // B22
     }
   }
   double lmax = (double)lm;
   asm volatile("" : "+v"(lmax));
-  FF::run_wide(w, t, X, twf, typename C::PF{});
-  if (t < NM * P * NB) {
+  FF::run(w, t, X, twf, typename C::PF{});
+  {
     unsigned tt = t;
     asm volatile("" : "+v"(tt));
     const unsigned s = tt / NB, j = tt % NB;
-    const unsigned pair = s / NM, m = s % NM;
+    const unsigned pair = s / 3, m = s % 3;
     const long la = line0 + 2 * pair, lb = la + 1;
     row_separate_store<T, NB, 24>(w, tt & 63, j, (vec2_t<T>*)(out + m * cs + la * a.ls),
                                   (vec2_t<T>*)(out + m * cs + lb * a.ls), cols);
@@ -1411,10 +1359,9 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
 // P = 768/L line pairs per 192-thread workgroup.  The inverse is the row-4
 // kernel's (3P packed sequences, 12 values per thread, plans 12.2.4.4 / 12.4.4;
 // at L = 384 its two middle passes run in half-waves, each sequence in its own
-// half-wave, so two of the three exchanges need no workgroup barrier); all
-// products of a pair (FP64 five, FP32 six, see products()) are formed at once and one forward
-// transform of as many sequences per pair (20 or 24 values per thread; with 20 the radix-24
-// pass on 160 threads, BlockFFT2::run_wide; plans 4.4.24 / 4.2.24, exchanges in real/imaginary
+// half-wave, so two of the three exchanges need no workgroup barrier); all six
+// products of a pair are formed at once and one 6P-sequence forward transform
+// (24 values per thread, plans 4.4.24 / 4.2.24, exchanges in real/imaginary
 // halves) replaces two rounds of 3P.  FP64 at L = 96 (P = 8, plans 12.2.4 / 4.24)
 // too: one forward exchange instead of four, 19.4 -> 17.2 us at 64^3, whose 576
 // workgroups are resident together although three, not four, fit a CU.  (FP32
@@ -1455,10 +1402,9 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   using FI = BlockFFT2<T, L, 3 * P, NT, +1, false, 3, MAP_SEQ1, MAP_SEQ, true, C::SOFFI, 0u, 0, C::MIDH>;
   // forward exchanges in real/imaginary halves: FP64 to fit four workgroups per
   // CU, FP32 (20 KB) to run four waves per SIMD
-  constexpr int NM = products<T, 3>();
-  using FF = BlockFFT2<T, L, NM * P, NT, -1, true, NM, MAP_SEQ, MAP_SEQ1, true, C::SOFFF, 0u,
+  using FF = BlockFFT2<T, L, 6 * P, NT, -1, true, 6, MAP_SEQ, MAP_SEQ1, true, C::SOFFF, 0u,
                        C::template fwd_pade<T>()>;
-  static_assert(FI::E == 12 && FF::E == 4 * NM, "thread layout");
+  static_assert(FI::E == 12 && FF::E == 24, "thread layout");
   constexpr int XWORDS = FI::lds_words > FF::lds_words ? FI::lds_words : FF::lds_words;
   static_assert((L == 96 ? 3 : 4) * (XWORDS * (int)sizeof(T) + 3 * 8) <= 163840, "workgroups per CU");
   __shared__ T X[XWORDS];
@@ -1496,32 +1442,26 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   asm volatile("" : "+v"(lmax));
 
   // products of this thread's pair (t / (L/4)) at its 4 positions: w[m*4 + r] =
-  // B_m (line a) + i B_m (line b), m = 0..5: B11, B21, B22, B31, B32, B33 (see products())
+  // B_m (line a) + i B_m (line b), m = 0..5: B11, B21, B22, B31, B32, B33
   cx<T> w[24];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const cx<T> p0 = u[r], p1 = u[4 + r], p2 = u[8 + r];
     const T a1 = nrm * p0.x, a2 = nrm * p0.y, a3 = nrm * p1.x;
     const T b1 = nrm * p2.x, b2 = nrm * p2.y, b3 = nrm * p1.y;
+    w[0 * 4 + r] = mk(a1 * a1, b1 * b1);
     w[1 * 4 + r] = mk(a2 * a1, b2 * b1);
+    w[2 * 4 + r] = mk(a2 * a2, b2 * b2);
     w[3 * 4 + r] = mk(a3 * a1, b3 * b1);
     w[4 * 4 + r] = mk(a3 * a2, b3 * b2);
-    if constexpr (NM == 5) {
-      const T a33 = a3 * a3, b33 = b3 * b3;
-      w[0 * 4 + r] = mk(a1 * a1 - a33, b1 * b1 - b33);
-      w[2 * 4 + r] = mk(a2 * a2 - a33, b2 * b2 - b33);
-    } else {
-      w[0 * 4 + r] = mk(a1 * a1, b1 * b1);
-      w[2 * 4 + r] = mk(a2 * a2, b2 * b2);
-      w[5 * 4 + r] = mk(a3 * a3, b3 * b3);
-    }
+    w[5 * 4 + r] = mk(a3 * a3, b3 * b3);
   }
-  FF::run_wide(w, t, X, tw, typename C::PF{});
-  if (t < NM * P * NBF) {
+  FF::run(w, t, X, tw, typename C::PF{});
+  {
     unsigned tt = t;
     asm volatile("" : "+v"(tt));
     const unsigned s = tt / NBF, j = tt % NBF;
-    const unsigned pair = s / NM, m = s % NM;
+    const unsigned pair = s / 6, m = s % 6;
     const long la = line0 + 2 * pair, lb = la + 1;
     row_separate_store<T, NBF, 24>(w, tt & 63, j, (vec2_t<T>*)(out + ((long)m * a.nlines + la) * a.ls),
                                    (vec2_t<T>*)(out + ((long)m * a.nlines + lb) * a.ls));

@@ -337,7 +337,6 @@ int enqueue_rhs_3d(azb_solver* s, const double2* u_in, const double2* u0, double
   const int N = s->N, M = s->M, nh = s->nh;
   const long S = s->S;
   const long hp = s->nhp;  // padded last-axis stride of every intermediate
-  constexpr int NM = products<T, 3>();
   hipStream_t st = s->stream;
   int rc;
   ColArgs c{};
@@ -373,7 +372,7 @@ int enqueue_rhs_3d(azb_solver* s, const double2* u_in, const double2* u0, double
   }
   // K3: last axis c2r, products, max, r2c; Y[c][line][hp] -> Z[m][line][hp]
   r.in = s->Y; r.out = s->Z; r.nlines = (long)M * M;
-  r.in_ss = 3L * M * M * hp; r.out_ss = (long)NM * M * M * hp;
+  r.in_ss = 3L * M * M * hp; r.out_ss = 6L * M * M * hp;
   {
     ProfScope p(s, AZB_PROF_ROW);
     if ((rc = launch_row<T, 3>(M, r, S, st, s->pdiv))) return rc;
@@ -383,20 +382,20 @@ int enqueue_rhs_3d(azb_solver* s, const double2* u_in, const double2* u0, double
   c.in_qs = 0; c.out_qs = 0;
   c.in_rs = hp; c.out_rs = hp;
   c.in_bs = (long)M * hp; c.out_bs = (long)N * hp;
-  c.bps = NM * M;
+  c.bps = 6 * M;
   {
     ProfScope p(s, AZB_PROF_FWD_AX1);
-    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, (long)NM * M * S, st, s->tsdiv[AZB_PROF_FWD_AX1], s->plan[AZB_PROF_FWD_AX1]))) return rc;
+    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 6L * M * S, st, s->tsdiv[AZB_PROF_FWD_AX1], s->plan[AZB_PROF_FWD_AX1]))) return rc;
   }
   // K5: forward along axis 0; X[m][i'][j][hp] -> Y[m][i][j][hp] (B_hat on the N-grid)
   c.in = s->X; c.out = s->Y; c.nq = N;
   c.in_qs = hp; c.out_qs = hp;
   c.in_rs = (long)N * hp; c.out_rs = (long)N * hp;
   c.in_bs = (long)M * N * hp; c.out_bs = (long)N * N * hp;
-  c.bps = NM;
+  c.bps = 6;
   {
     ProfScope p(s, AZB_PROF_FWD_AX0);
-    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, (long)NM * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
+    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 6L * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
   }
   const double Md = std::pow((double)M, 3);
   KArgs k{};
@@ -467,7 +466,7 @@ int enqueue_row_2d(azb_solver* s, int slot, bool begin, long ls, int bw, long co
   r.bw = bw;
   r.norm = 1.0 / (std::pow(std::sqrt((double)N), 2) * std::pow(std::sqrt((double)M), 2));
   r.in = s->X; r.out = s->Z; r.nlines = M;
-  r.in_ss = 2 * comp; r.out_ss = products<T, 2>() * comp;
+  r.in_ss = 2 * comp; r.out_ss = 3 * comp;
   ProfScope p(s, AZB_PROF_ROW);
   return launch_row<T, 2>(M, r, s->S, s->stream);
 }
@@ -551,10 +550,10 @@ int enqueue_rhs_2d_passes(azb_solver* s, const double2* u_in, const double2* u0,
   c.in = s->Z; c.out = s->Y;
   c.in_rs = hp; c.out_rs = hp;
   c.in_bs = (long)M * hp; c.out_bs = (long)N * hp;
-  c.bps = products<T, 2>();
+  c.bps = 3;
   {
     ProfScope p(s, AZB_PROF_FWD_AX0);
-    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, (long)products<T, 2>() * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
+    if ((rc = launch_col<T, T, T, -1, COL_TRUNC_OUT>(M, c, 3L * S, st, s->tsdiv[AZB_PROF_FWD_AX0], s->plan[AZB_PROF_FWD_AX0]))) return rc;
   }
   KArgs k{};
   // the max|u| reduction runs inside the k-space kernel (a launch less per RHS where
@@ -628,14 +627,9 @@ int check_solver_args(int dim, int N, int M, int n_vars, int precision, int nsam
   return AZB_OK;
 }
 
-size_t num_products(int precision, int dim) {
-  const int all = 3 * (dim - 1);
-  return all - (precision == AZB_FP64 ? 1 : 0);
-}
-
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
-size_t bhat_bytes_2d(const azb_solver* s) { return (size_t)s->S * 2 * s->tsize * num_products(s->prec, 2) * (size_t)s->N * s->nhp; }
+size_t bhat_bytes_2d(const azb_solver* s) { return (size_t)s->S * 2 * s->tsize * 3 * (size_t)s->N * s->nhp; }
 
 // bytes of the intermediates X, Y, Z and of one RK stage buffer for S samples
 struct Layout {
@@ -677,14 +671,13 @@ Layout setup_solver(azb_solver* s, int dim, int N, int precision, azb_sv_params 
   Layout l{};
   if (dim == 3) {
     s->nmodes = (long)N * N * nh;
-    const size_t nm = num_products(precision, 3);
-    l.xs = S * cs * nm * (size_t)M * N * hp;                                   // T1 (3) / S2
-    l.ys = S * cs * std::max<size_t>(3 * (size_t)M * M * hp, nm * (size_t)N * N * hp);  // T2 / B_hat
-    l.zs = S * cs * nm * (size_t)M * M * hp;                                   // S1
+    l.xs = S * cs * 6 * (size_t)M * N * hp;                                   // T1 (3) / S2 (6)
+    l.ys = S * cs * std::max<size_t>(3 * (size_t)M * M * hp, 6 * (size_t)N * N * hp);  // T2 / B_hat
+    l.zs = S * cs * 6 * (size_t)M * M * hp;                                   // S1
   } else {
     s->nmodes = (long)N * nh;
     l.xs = S * cs * 2 * (size_t)M * hp;
-    l.zs = S * cs * num_products(precision, 2) * (size_t)M * hp;
+    l.zs = S * cs * 3 * (size_t)M * hp;
     s->stage = stage_shape((int)s->tsize, M, nsamples);
     if (s->stage.width) l.ms = sizeof(double2) * s->nmodes;
     // B_hat exists only between separate passes
@@ -813,14 +806,13 @@ int azb_num_samples(const azb_solver* s) { return s ? s->S : 0; }
 size_t azb_bytes_estimate(int dim, int N, int precision, int nsamples) {
   const size_t cs = precision == AZB_FP64 ? 16 : 8;
   const size_t M = 3 * (size_t)N / 2, nh = N / 2 + 1, hp = (nh + 15) / 16 * 16, S = nsamples;
-  const size_t nm = num_products(precision, dim);
   size_t ws, us, ms = 0;
   if (dim == 3) {
-    ws = cs * (nm * M * N * hp + std::max(3 * M * M * hp, nm * N * N * hp) + nm * M * M * hp);
+    ws = cs * (6 * M * N * hp + std::max(3 * M * M * hp, 6 * (size_t)N * N * hp) + 6 * M * M * hp);
     us = sizeof(double2) * 3 * (size_t)N * N * nh;
   } else {
     const size_t w = stage_shape(precision == AZB_FP64 ? 8 : 4, (int)M, nsamples).width;
-    ws = cs * (2 * M * hp + (w && !rhs_alone_separate(N) ? 0 : nm * N * hp) + nm * M * hp);
+    ws = cs * (2 * M * hp + (w && !rhs_alone_separate(N) ? 0 : 3 * (size_t)N * hp) + 3 * M * hp);
     us = sizeof(double2) * 2 * (size_t)N * (w ? (nh + w - 1) / w * w : nh);
     ms = w ? sizeof(double2) * (size_t)N * nh : 0;
   }

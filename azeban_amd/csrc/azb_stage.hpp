@@ -2,7 +2,7 @@
 //
 // In 2D the axis-0 transforms of one block of last-axis modes k touch nothing but that
 // block, so one workgroup takes TS consecutive k and runs for them
-//   forward  : the products' axis-0 transforms (M rows in, the N kept ones used),
+//   forward  : the three products' axis-0 transforms (M rows in, the N kept ones used),
 //   k-space  : ik.B_hat, Leray, viscosity and the RK stage update of every mode (i, k),
 //   inverse  : the axis-0 transforms of the two components of the new stage value, the
 //              next row kernel's input.
@@ -17,7 +17,7 @@ namespace azb {
 // contiguous run per component, and the TS modes of the consecutive lines that a row
 // workgroup holds lie next to each other, so both kernels move whole cache lines.
 struct StageArgs {
-  const void* s2;       // [sample][products][block][M][TS] products after the row kernel, working precision
+  const void* s2;       // [sample][3][block][M][TS] products after the row kernel, working precision
   const double2* u_in;  // stage input u_hat
   const double2* u0;    // RK base state (stages 2, 3), in the caller's layout [sample][2][N][nh]
   double2* out;         // stage value (or du/dt)
@@ -47,9 +47,8 @@ struct StageCfg {
   static constexpr int NT = F * TS * L / 8;
   static constexpr int N = 2 * L / 3;
   using P = typename LenPlan<L>::P;
-  static constexpr int NM = products<T, 2>();
+  using LF = ColLayout<3 * TS, 2 * TS>;
   using LI = ColLayout<2 * TS, TS>;
-  using LF = std::conditional_t<NM == 2, LI, ColLayout<3 * TS, 2 * TS>>;
   static constexpr int ELEMS = LF::elems(L);
   // real and imaginary halves in turn unless whole values leave room for four (FP32: two) workgroups
   static constexpr bool SPLIT = ELEMS * 2 * (int)sizeof(T) > (sizeof(T) == 8 ? 40960 : 81920);
@@ -63,9 +62,9 @@ template <typename T, int L, int TS, int F>
 __global__ __launch_bounds__((StageCfg<T, L, TS, F>::NT)) __attribute__((amdgpu_waves_per_eu(3))) void col_stage_kernel(StageArgs a) {
   using C = StageCfg<T, L, TS, F>;
   using P = typename C::P;
-  constexpr int NT = C::NT, N = C::N, half = N / 2, RL = last_radix(P{}), NQ = 2 / F, NM = C::NM;
+  constexpr int NT = C::NT, N = C::N, half = N / 2, RL = last_radix(P{}), NQ = 2 / F;
   constexpr bool SPLIT = C::SPLIT, PT = sizeof(T) == 4 && L == 768;
-  using FF = ColFFT<T, L, NM * TS, NT, -1, SPLIT, typename C::LF, PT>;
+  using FF = ColFFT<T, L, 3 * TS, NT, -1, SPLIT, typename C::LF, PT>;
   using FI = ColFFT<T, L, 2 * TS, NT, +1, SPLIT, typename C::LI, PT>;
   using LF = typename C::LF;
   using LI = typename C::LI;
@@ -82,8 +81,8 @@ __global__ __launch_bounds__((StageCfg<T, L, TS, F>::NT)) __attribute__((amdgpu_
 
   cx<T> v[24];
   if (!lead) {
-    const void* in = (const cx<T>*)a.s2 + sample * ((long)NM * cs) + kt * (L * TS);
-    const unsigned s = t % (unsigned)(NM * TS), m = s / TS, col = s % TS, j = t / (unsigned)(NM * TS);
+    const void* in = (const cx<T>*)a.s2 + sample * (3l * cs) + kt * (L * TS);
+    const unsigned s = t % (3u * TS), m = s / TS, col = s % TS, j = t / (3u * TS);
     const unsigned base = m * cs + j * TS + col;
 #pragma unroll
     for (int b = 0; b < FF::template rounds<8>(); ++b)
@@ -176,12 +175,11 @@ __global__ __launch_bounds__((StageCfg<T, L, TS, F>::NT)) __attribute__((amdgpu_
 #pragma unroll
       for (int q = 0; q < NQ; ++q) w[8 * q + radix_row(e)] = mk(T(u[q][e].x), T(u[q][e].y));
   } else {
-    constexpr int NB = dot_values<2, NM>();
-    double br[NB][NE];  // real half of b = ik.B_hat
+    double br[2][NE];  // real half of b = ik.B_hat
     const double2* modes = a.modes + c0;
     double2* out = a.out + (a.out_blocked ? bbase : sbase);
     auto put_kept = [&](int c) {  // kept rows of the forward output, half c
-      const unsigned s = tt % (unsigned)(NM * TS), j0 = tt / (unsigned)(NM * TS);
+      const unsigned s = tt % (3u * TS), j0 = tt / (3u * TS);
 #pragma unroll
       for (int b = 0; b < FF::template rounds<RL>(); ++b)
 #pragma unroll
@@ -204,15 +202,15 @@ __global__ __launch_bounds__((StageCfg<T, L, TS, F>::NT)) __attribute__((amdgpu_
     };
     auto real_half = [&](int e) {  // from the imaginary parts
       if (!keep[e]) return;
-      double B[NM], o[NB];
+      double B[3], o[2];
 #pragma unroll
-      for (int m = 0; m < NM; ++m) {
+      for (int m = 0; m < 3; ++m) {
         const unsigned idx = LF::at(m * TS + col, j + radix_row(e) * (L / 8));
         B[m] = -(double)lds[SPLIT ? idx : 2 * idx + 1];
       }
-      kspace_dot<2, NM>(mode_of(e, 0.0), B, o);
-#pragma unroll
-      for (int q = 0; q < NB; ++q) br[q][e] = o[q];
+      kspace_dot<2>(mode_of(e, 0.0), B, o);
+      br[0][e] = o[0];
+      br[1][e] = o[1];
     };
     __syncthreads();
     put_kept(1);
@@ -251,17 +249,16 @@ __global__ __launch_bounds__((StageCfg<T, L, TS, F>::NT)) __attribute__((amdgpu_
         if (!SPLIT) real_half(e);
         if (!keep[e]) continue;
         const ModeGeom<2> g = mode_of(e, md[i].x);
-        double B[NM], b2[NB], bi[NB], Lr[2], Li[2];
+        double B[3], bi[2], Lr[2], Li[2];
+        const double b2[2] = {br[0][e], br[1][e]};
 #pragma unroll
-        for (int q = 0; q < NB; ++q) b2[q] = br[q][e];
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
+        for (int m = 0; m < 3; ++m) {
           const unsigned idx = LF::at(m * TS + col, j + radix_row(e) * (L / 8));
           B[m] = (double)lds[SPLIT ? idx : 2 * idx];
         }
-        kspace_dot<2, NM>(g, B, bi);
-        kspace_project<2, NM>(g, b2, Lr);
-        kspace_project<2, NM>(g, bi, Li);
+        kspace_dot<2>(g, B, bi);
+        kspace_project<2>(g, b2, Lr);
+        kspace_project<2>(g, bi, Li);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
           const double lr = F == 1 ? Lr[q] : (q0 == 0 ? Lr[0] : Lr[1]);

@@ -4,8 +4,7 @@ Bytes = logical elements a kernel must read + elements it must write, at storage
 precision, each counted once; implicit zero padding and truncated modes are not
 counted.  Complex state (u_hat, RK buffers): 16 B; intermediates: 16 B (FP64) or
 8 B (FP32-mixed).  2D: one sample per solver (the column stage).  N: grid,
-M = 3N/2, nh = N/2 + 1.  The products transformed back: dim(dim+1)/2, less one
-in FP64 (the last diagonal one is taken off the others).
+M = 3N/2, nh = N/2 + 1, nb = dim(dim+1)/2 products.
 """
 from __future__ import annotations
 
@@ -15,7 +14,7 @@ def family_bytes(dim: int, N: int, precision: str = "fp64") -> dict:
     nh = N // 2 + 1
     cs = 16 if precision == "fp64" else 8
     S = 16
-    nb = dim * (dim + 1) // 2 - (precision == "fp64")
+    nb = dim * (dim + 1) // 2
     if dim == 3:
         nm = N * N * nh
         fam = {
