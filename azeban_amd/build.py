@@ -25,7 +25,7 @@ UNITS = [
 ]
 SOURCES = [u[0] for u in UNITS]
 HEADERS = [CSRC / "azb_fft.hpp", CSRC / "azb_kernels.hpp", CSRC / "azb_aux_kernels.hpp", CSRC / "azb_launch.hpp",
-           CSRC / "azb_stage.hpp", CSRC / "azb_seam_fft.hpp",
+           CSRC / "azb_stage.hpp", CSRC / "azb_seam_fft.hpp", CSRC / "azb_slots.hpp",
            ROOT / "include" / "azeban_hip.h"]
 
 HIPCC_FLAGS = [

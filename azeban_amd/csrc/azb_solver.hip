@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -16,6 +17,7 @@
 #include "azb_kernels.hpp"
 #include "azb_launch.hpp"
 #include "azb_seam_fft.hpp"
+#include "azb_slots.hpp"
 
 using namespace azb;
 
@@ -1503,54 +1505,66 @@ constexpr size_t kFftSlotsBytes = size_t(256) << 10;
 // Small device results of the synchronising reductions (energy spectrum, max norm): a call
 // takes one of the file-scope slots for its duration instead of allocating, or allocates
 // when all are taken or its result is longer.
-constexpr int kResultSlots = 16, kResultLen = 1024;
-static __device__ double result_slots[kResultSlots * kResultLen];
+constexpr int kResultLen = 1024;
+static __device__ double result_slots[SlotSet::kSlots * kResultLen];
 static __device__ __align__(256) unsigned char fft_slots[kFftSlotsBytes];
 
 namespace {
 
-std::mutex g_result_mu;
-struct ResultSlots {
-  double* base = nullptr;
-  unsigned taken = 0;
+// The calls below wait for their stream, so they cannot be part of a capture; refused before
+// anything is queued, which leaves the capture as it was.
+int not_capturing(hipStream_t st) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return AZB_OK;
+  }
+  return status == hipStreamCaptureStatusNone ? AZB_OK
+                                              : fail(AZB_ERR_HIP, "the stream is being captured, the call waits for it");
+}
+
+struct StreamWait {
+  hipStream_t st;
+  int operator()() const { return (int)hipStreamSynchronize(st); }
 };
-std::vector<ResultSlots> g_result_slots;  // per device
+
+struct DeviceSlots {
+  double* base = nullptr;
+  SlotSet set;
+};
+std::mutex g_result_mu;
+std::vector<std::unique_ptr<DeviceSlots>> g_result_slots;  // per device
 
 struct ResultSlot {
   double* p = nullptr;
-  int dev = -1, index = -1;
   DevFree own;
-  ResultSlot() = default;
-  ResultSlot(const ResultSlot&) = delete;
-  ResultSlot& operator=(const ResultSlot&) = delete;
+  SlotLease<StreamWait> lease;
+  explicit ResultSlot(hipStream_t st) : lease(StreamWait{st}) {}
   int get(int n) {
-    HIPCHK(hipGetDevice(&dev));
     if (n <= kResultLen) {
-      std::lock_guard<std::mutex> lock(g_result_mu);
-      if ((int)g_result_slots.size() <= dev) g_result_slots.resize(dev + 1);
-      ResultSlots& d = g_result_slots[dev];
-      if (!d.base) {
-        void* a = nullptr;
-        HIPCHK(hipGetSymbolAddress(&a, HIP_SYMBOL(result_slots)));
-        d.base = (double*)a;
+      int dev = -1;
+      HIPCHK(hipGetDevice(&dev));
+      DeviceSlots* d;
+      {
+        std::lock_guard<std::mutex> lock(g_result_mu);
+        if ((int)g_result_slots.size() <= dev) g_result_slots.resize(dev + 1);
+        if (!g_result_slots[dev]) {
+          void* a = nullptr;
+          HIPCHK(hipGetSymbolAddress(&a, HIP_SYMBOL(result_slots)));
+          g_result_slots[dev] = std::make_unique<DeviceSlots>();
+          g_result_slots[dev]->base = (double*)a;
+        }
+        d = g_result_slots[dev].get();
       }
-      for (int i = 0; i < kResultSlots && index < 0; ++i)
-        if (!(d.taken >> i & 1)) index = i;
-      if (index >= 0) {
-        d.taken |= 1u << index;
-        p = d.base + index * kResultLen;
+      const int i = lease.take(d->set);
+      if (i >= 0) {
+        p = d->base + i * kResultLen;
         return AZB_OK;
       }
     }
     HIPCHK(hipMalloc(&own.p, sizeof(double) * n));
     p = (double*)own.p;
     return AZB_OK;
-  }
-  // the owner has waited for its stream, or that wait failed and the device is lost
-  ~ResultSlot() {
-    if (index < 0) return;
-    std::lock_guard<std::mutex> lock(g_result_mu);
-    g_result_slots[dev].taken &= ~(1u << index);
   }
 };
 
@@ -1726,10 +1740,12 @@ int azb_energy_spectrum(int dim, int N, const void* u_hat, double* spec_host, vo
   hipStream_t st = (hipStream_t)stream;
   const long nh = N / 2 + 1;
   const long nmodes = dim == 2 ? (long)N * nh : (long)N * N * nh;
-  ResultSlot slot;
-  int rc = slot.get((int)nh);
+  int rc = not_capturing(st);
   if (rc) return rc;
+  ResultSlot slot(st);
+  if ((rc = slot.get((int)nh))) return rc;
   double* d = slot.p;
+  slot.lease.queued();
   hipLaunchKernelGGL(zero_kernel, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, st, d, (int)nh);
   const long rows = dim == 2 ? N : (long)N * N;
   const unsigned blocks = (unsigned)std::min<long>((rows + 3) / 4, 2048);
@@ -1741,7 +1757,7 @@ int azb_energy_spectrum(int dim, int N, const void* u_hat, double* spec_host, vo
                        (const double2*)u_hat, N, nmodes, d);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(spec_host, d, sizeof(double) * nh, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
+  HIPCHK((hipError_t)slot.lease.wait());
   return AZB_OK;
 }
 
@@ -1757,9 +1773,11 @@ int azb_axpby(double a, const void* x, double b, void* y, long n, void* stream) 
 int azb_max_norm(const void* x, long n, double* out_host, void* stream) {
   if (!x || !out_host) return fail(AZB_ERR_ARG, "NULL argument");
   hipStream_t st = (hipStream_t)stream;
-  ResultSlot slot;
-  int rc = slot.get(1);
+  int rc = not_capturing(st);
   if (rc) return rc;
+  ResultSlot slot(st);
+  if ((rc = slot.get(1))) return rc;
+  slot.lease.queued();
   unsigned long long* d = (unsigned long long*)slot.p;
   hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, st, slot.p, 1);
   if (n > 0) {
@@ -1769,7 +1787,7 @@ int azb_max_norm(const void* x, long n, double* out_host, void* stream) {
   }
   unsigned long long bits = 0;
   HIPCHK(hipMemcpyAsync(&bits, d, sizeof(bits), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
+  HIPCHK((hipError_t)slot.lease.wait());
   double v;
   std::memcpy(&v, &bits, sizeof(v));
   *out_host = v;
