@@ -56,6 +56,16 @@ __global__ void loop_set_all(DevState* st_all, int nsamples, double time, double
   st->steps = 0;
 }
 
+// what the host reads of a sample's loop, stored where it can (pinned memory)
+struct LoopReport {
+  double time;
+  long steps;
+};
+__global__ void loop_report(const DevState* st, int nsamples, LoopReport* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nsamples) out[i] = LoopReport{st[i].time, (long)st[i].steps};
+}
+
 // (re)start the device-driven loop of one sample: its time, target and step count
 __global__ void loop_set_sample(DevState* st_all, int sample, double time, double t_end, double max_dt_visc) {
   if (threadIdx.x != 0) return;

@@ -49,6 +49,56 @@ struct DevFree {
   }
 };
 
+// Calls that wait for their stream cannot be part of a capture; refused before anything is
+// queued, which leaves the capture as it was.
+int not_capturing(hipStream_t st) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return AZB_OK;
+  }
+  return status == hipStreamCaptureStatusNone ? AZB_OK
+                                              : fail(AZB_ERR_HIP, "the stream is being captured, the call waits for it");
+}
+
+struct StreamWait {
+  hipStream_t st;
+  int operator()() const { return (int)hipStreamSynchronize(st); }
+};
+
+// Where kernels store what a call returns to the host: pinned slots of one array per process,
+// made with the first solver and held until the process ends.  A call takes one for its
+// duration; allocating them per solver cost its first step 30 us (64^2: 93 instead of 63).
+constexpr int kPinnedLen = 1024;  // entries per slot
+SlotSet g_pinned_set;
+
+LoopReport* pinned_slots() {
+  static std::mutex mu;
+  static LoopReport* base = nullptr;
+  std::lock_guard<std::mutex> lock(mu);
+  if (!base) {
+    void* p = nullptr;
+    // every device may write to it, and its stores need no flush to be seen after a wait
+    if (hipHostMalloc(&p, sizeof(LoopReport) * kPinnedLen * SlotSet::kSlots,
+                      hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess)
+      base = (LoopReport*)p;
+    else
+      (void)hipGetLastError();
+  }
+  return base;
+}
+
+struct PinnedSlot {
+  SlotLease<StreamWait> lease;
+  explicit PinnedSlot(hipStream_t st) : lease(StreamWait{st}) {}
+  // a slot for n entries, or NULL (all taken, n too large, no pinned memory): the caller copies instead
+  LoopReport* get(int n) {
+    LoopReport* base = n <= kPinnedLen ? pinned_slots() : nullptr;
+    const int i = base ? lease.take(g_pinned_set) : -1;
+    return i < 0 ? nullptr : base + i * kPinnedLen;
+  }
+};
+
 bool good_len(int L) {
   switch (L) {
     case 48: case 96: case 192: case 384: case 768: case 1536:
@@ -287,9 +337,7 @@ struct azb_solver {
   // radix plan per column-pass family (ColPlan index; the row and k-space entries are 0)
   int plan[AZB_PROF_FAMILIES] = {0, 0, 0, 0, 0, 0};
   StageShape stage{0, 0};  // 2D column stage; width 0: separate passes
-  double* dt_host = nullptr;  // pinned, written by the kernels of a fixed step that reports its dt
-  double* dt_out = nullptr;   // dt_host while such a step is queued
-  DevState* read_host = nullptr;  // pinned mirror of the device state (blocking reads)
+  double* dt_out = nullptr;  // pinned, while a step that reports its dt is queued
   DevState* probe_host = nullptr;  // pinned mirror of the device state (non-blocking probes)
   hipEvent_t probe_ev = nullptr;
   // per-kernel-family hipEvent timing (off unless enabled)
@@ -765,6 +813,7 @@ int azb_create_batch(int dim, int N, int M, int n_vars, int precision, azb_sv_pa
   *out = nullptr;
   int rc = check_solver_args(dim, N, M, n_vars, precision, nsamples);
   if (rc) return rc;
+  (void)pinned_slots();
   azb_solver* s = new azb_solver();
   const Layout lay = setup_solver(s, dim, N, precision, visc, nsamples);
   const size_t xs = lay.xs, ys = lay.ys, zs = lay.zs, us = lay.us, ms = lay.ms, S = nsamples;
@@ -831,8 +880,6 @@ int azb_destroy(azb_solver* s) {
   (void)hipFree(s->u2);
   (void)hipFree(s->st);
   (void)hipFree(s->tw);
-  if (s->dt_host) (void)hipHostFree(s->dt_host);
-  if (s->read_host) (void)hipHostFree(s->read_host);
   if (s->probe_host) (void)hipHostFree(s->probe_host);
   if (s->probe_ev) (void)hipEventDestroy(s->probe_ev);
   for (auto& e : s->prof_ev) {
@@ -906,16 +953,22 @@ int azb_dt(azb_solver* s, double C, double* dt_host) {
 
 int azb_rk3_step(azb_solver* s, void* u_hat, double max_dt, double C, double* dt_host) {
   if (!s || !u_hat) return fail(AZB_ERR_ARG, "NULL argument");
-  if (dt_host && !s->dt_host) HIPCHK(hipHostMalloc((void**)&s->dt_host, sizeof(double), hipHostMallocDefault));
-  hipLaunchKernelGGL(step_prologue_fixed, dim3(s->S), dim3(256), 0, s->stream, s->st, max_dt);
+  int rc;
+  if (dt_host && (rc = not_capturing(s->stream))) return rc;
+  PinnedSlot slot(s->stream);
   // the kernel that takes dt also stores it where the host reads it: no copy to wait for
-  s->dt_out = dt_host ? s->dt_host : nullptr;
-  int rc = enqueue_rk3_stages(s, (double2*)u_hat, C);
+  double* out = dt_host ? (double*)slot.get(1) : nullptr;
+  slot.lease.queued();
+  hipLaunchKernelGGL(step_prologue_fixed, dim3(s->S), dim3(256), 0, s->stream, s->st, max_dt);
+  s->dt_out = out;
+  rc = enqueue_rk3_stages(s, (double2*)u_hat, C);
   s->dt_out = nullptr;
   if (rc) return rc;
   if (dt_host) {
-    HIPCHK(hipStreamSynchronize(s->stream));
-    *dt_host = *s->dt_host;
+    double dt = 0.0;
+    if (!out) HIPCHK(hipMemcpyAsync(&dt, &s->st->dt, sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    HIPCHK((hipError_t)slot.lease.wait());
+    *dt_host = out ? *out : dt;
   }
   return AZB_OK;
 }
@@ -973,13 +1026,24 @@ int azb_enqueue_steps(azb_solver* s, void* u_hat, int nsteps) {
 
 int azb_loop_read(azb_solver* s, double* times_host, int* steps_host) {
   if (!s) return fail(AZB_ERR_ARG, "NULL solver");
-  if (!s->read_host)
-    HIPCHK(hipHostMalloc((void**)&s->read_host, s->S * sizeof(DevState), hipHostMallocDefault));
-  HIPCHK(hipMemcpyAsync(s->read_host, s->st, s->S * sizeof(DevState), hipMemcpyDeviceToHost, s->stream));
-  HIPCHK(hipStreamSynchronize(s->stream));
+  int rc = not_capturing(s->stream);
+  if (rc) return rc;
+  PinnedSlot slot(s->stream);
+  const LoopReport* out = slot.get(s->S);
+  std::vector<DevState> copy;
+  if (out) {
+    slot.lease.queued();
+    hipLaunchKernelGGL(loop_report, dim3((unsigned)((s->S + 63) / 64)), dim3(64), 0, s->stream, s->st, s->S,
+                       (LoopReport*)out);
+    HIPCHK(hipGetLastError());
+  } else {
+    copy.resize(s->S);
+    HIPCHK(hipMemcpyAsync(copy.data(), s->st, s->S * sizeof(DevState), hipMemcpyDeviceToHost, s->stream));
+  }
+  HIPCHK((hipError_t)slot.lease.wait());
   for (int i = 0; i < s->S; ++i) {
-    if (times_host) times_host[i] = s->read_host[i].time;
-    if (steps_host) steps_host[i] = s->read_host[i].steps;
+    if (times_host) times_host[i] = out ? out[i].time : copy[i].time;
+    if (steps_host) steps_host[i] = out ? (int)out[i].steps : copy[i].steps;
   }
   return AZB_OK;
 }
@@ -1510,23 +1574,6 @@ static __device__ double result_slots[SlotSet::kSlots * kResultLen];
 static __device__ __align__(256) unsigned char fft_slots[kFftSlotsBytes];
 
 namespace {
-
-// The calls below wait for their stream, so they cannot be part of a capture; refused before
-// anything is queued, which leaves the capture as it was.
-int not_capturing(hipStream_t st) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &status) != hipSuccess) {
-    (void)hipGetLastError();
-    return AZB_OK;
-  }
-  return status == hipStreamCaptureStatusNone ? AZB_OK
-                                              : fail(AZB_ERR_HIP, "the stream is being captured, the call waits for it");
-}
-
-struct StreamWait {
-  hipStream_t st;
-  int operator()() const { return (int)hipStreamSynchronize(st); }
-};
 
 struct DeviceSlots {
   double* base = nullptr;

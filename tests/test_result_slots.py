@@ -54,3 +54,54 @@ def test_reductions_are_refused_under_capture(cuda):
         np.testing.assert_allclose(A.energy_spectrum(u), spectrum, rtol=1e-13)
     _capi.check(lib.azb_graph_destroy(graph))
     _capi.check(lib.azb_stream_destroy(st))
+
+
+def _mappings():
+    with open("/proc/self/maps") as f:
+        return sum(1 for _ in f)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim", [2, 3])
+def test_first_calls_of_a_new_solver_allocate_nothing(cuda, dim):
+    """A solver's first step and its first run take as long as the later ones: what they return goes
+    through memory that is there.  A pinned allocation shows as a mapping of its own."""
+    import math
+
+    import azeban_amd as A
+
+    g = A.Grid(dim, 64)
+    rng = np.random.default_rng(5)
+    u = A.initialize(rng.standard_normal((dim,) + (64,) * dim))
+    grown = []
+    for i in range(4):  # the first solver warms the process up
+        eq = A.IncompressibleEuler(g, A.SmoothCutoff1D(0.05 / 64, 1.0, 2 * math.pi * 16))
+        step = A.SSP_RK3(u.shape, eq)
+        sim = A.Simulation(g, 0.2, step, u)
+        v = u.clone()
+        torch.cuda.synchronize()
+        print(f"[case] dim={dim} solver {i}", flush=True)
+        before = _mappings()
+        dt = step.integrate(1e6, 1e-3, 0.2, v)
+        assert sim.simulate_until(1e6, max_steps=2) == 2
+        grown.append(_mappings() - before)
+        assert 0 < dt <= 1e-3 and sim.time() > 0
+    assert grown[1:] == [0, 0, 0], grown
+
+
+@pytest.mark.gpu
+def test_loop_read_of_more_samples_than_a_slot_holds(cuda):
+    """1024 samples are reported through one slot, more are copied: the same times and steps either way."""
+    from azeban_amd.ensemble import Ensemble, Group
+
+    import azeban_amd as A
+
+    rng = np.random.default_rng(6)
+    one = A.initialize(rng.standard_normal((2, 64, 64)))
+    for S in (1024, 1025):
+        print(f"[case] {S} samples", flush=True)
+        ens = Ensemble([Group(2, 64, one.unsqueeze(0).repeat(S, 1, 1, 1), "fp64")], 0.2)
+        res = ens.run(1e6, steps_per_launch=2, max_launches=1)
+        t = ens.times()[0]
+        assert res["steps"] == [[2] * S] and len(set(t)) == 1 and t[0] > 0
+        ens.close()
