@@ -229,11 +229,13 @@ _PLANS: dict = {}
 def _ensure_plans(handle, dim: int, N: int, precision: str, u_hat: torch.Tensor, reps: int,
                   cache: str | None) -> list:
     """Give the solver the plans of its grid: from this process, from `cache`, or timed
-    now on the device (azb_autotune_plans) and remembered."""
+    now on the device (azb_autotune_plans) and remembered.  2D solvers have one choice, plan 0 of
+    the fused column stage; another one in a file of an earlier version, where the passes were
+    separate, would take them back to those (512^2: 137 us a step instead of 104)."""
     lib = load()
     key = f"{dim}/{N}/{precision}"
     plans = _PLANS.get(key)
-    if plans is None and cache:
+    if plans is None and cache and dim == 3:
         plans = _tuning_load(cache).get("plans", {}).get(key)
     n = len(_capi.PROF_FAMILIES)
     if plans is None:
