@@ -1464,7 +1464,7 @@ namespace {
 constexpr size_t kFftTwOffset = (sizeof(DevState) + 255) / 256 * 256;
 
 template <typename T>
-size_t fft_work_bytes(int n) {
+constexpr size_t fft_work_bytes(int n) {
   return kFftTwOffset + (sizeof(cx<T>) * (size_t)n + 255) / 256 * 256;
 }
 
@@ -1553,7 +1553,8 @@ int fft_c2r_T(int dim, int n, int howmany, double scale, const void* in, void* t
 // copy for the life of the process; a slot is written once, on its first use on a device.
 constexpr int kFftLens[13] = {16, 32, 48, 64, 96, 128, 192, 256, 384, 512, 768, 1024, 1536};
 
-size_t fft_slot_offset(int n, int precision) {
+// n = 0: the bytes of all slots
+constexpr size_t fft_slot_offset(int n, int precision) {
   size_t off = 0;
   for (int p : {AZB_FP64, AZB_FP32_MIXED})
     for (int L : kFftLens) {
@@ -1563,6 +1564,7 @@ size_t fft_slot_offset(int n, int precision) {
   return off;
 }
 constexpr size_t kFftSlotsBytes = size_t(256) << 10;
+static_assert(fft_slot_offset(0, AZB_FP64) <= kFftSlotsBytes, "a slot for every built length and precision");
 
 }  // namespace
 
