@@ -404,7 +404,7 @@ def fft_c2r(u_hat: torch.Tensor, n: int) -> torch.Tensor:
     """Unnormalised C2R; u_hat is left as it is."""
     _need("fft_c2r", u_hat, (torch.complex128, torch.complex64), _c2r_shape_ok(n),
           _C2R_SHAPE.format(n=n, nh=n // 2 + 1))
-    return _c2r(u_hat.resolve_conj().contiguous(), n, 1.0, False)
+    return _c2r(u_hat.resolve_conj().resolve_neg().contiguous(), n, 1.0, False)
 
 
 def leray_(u_hat: torch.Tensor) -> torch.Tensor:
@@ -484,7 +484,7 @@ def to_physical(u_hat: torch.Tensor, N_out: int | None = None) -> torch.Tensor:
     if n > N:
         raise ValueError("N_out must not exceed the grid size")
     _need("to_physical", u_hat, (torch.complex128,))
-    u_hat = u_hat.resolve_conj()
+    u_hat = u_hat.resolve_conj().resolve_neg()
     if n < N:
         u_hat = torch.stack([copy_from_padded(u_hat[c], n) for c in range(u_hat.shape[0])])
     _need("to_physical", u_hat, (torch.complex128,), _c2r_shape_ok(n), _C2R_SHAPE.format(n=n, nh=n // 2 + 1))
