@@ -226,7 +226,7 @@ struct RowArgs {
 // 2D: whether this workgroup's sample sits the launch out.  In the first kernel of a loop step
 // every workgroup decides from the sample's time, which no kernel of the previous step
 // still writes, and the sample's first workgroup records the decision and the step's clamp
-// for the kernels that follow (step_prologue_loop's work without its launch).
+// for the kernels that follow (step_control_loop's work without its launch).
 __device__ __forceinline__ bool row_idle(const RowArgs& a, DevState* st, bool first) {
   if (!a.begin) return st->done != 0;
   const bool go = st->time < st->t_end;
