@@ -13,6 +13,16 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "slow: long-running case")
 
 
+# Needs requests that arrive 0.5 ms apart to overlap, and a 64^2 request takes 0.2-0.3 ms in a
+# warm process: it runs last, so that a run that stops at its failure has run all the others
+# (test_slots_are_reused_when_all_requests_wait tests the same with equal arrivals).
+DEPENDS_ON_SOLVE_TIME = ("test_gpu_serving.py::test_slots_are_reused_by_later_requests",)
+
+
+def pytest_collection_modifyitems(items):
+    items.sort(key=lambda item: item.nodeid.endswith(DEPENDS_ON_SOLVE_TIME))
+
+
 @pytest.fixture(scope="session")
 def cuda():
     import torch

@@ -135,3 +135,24 @@ def test_one_at_a_time_baseline_gives_the_same_results(cuda):
     for res in srv.results:
         assert res.steps == got[res.rid].steps
         assert torch.equal(res.u_hat, got[res.rid].u_hat), res.rid
+
+
+def test_slots_are_reused_when_all_requests_wait(cuda):
+    """Seven requests for two slots, all there from the start: both slots are in use together however
+    fast a request is solved, and five requests join the batch in slots that others left."""
+    print("[case] serving slot reuse, equal arrivals", flush=True)
+    rs = []
+    for i in range(7):
+        u = initialize(I.fractional_brownian(2, 64, seed=300 + i))
+        rs.append(Request(i, 2, 64, u, 0.004 + 0.003 * (i % 3), 0.0))
+    torch.cuda.synchronize()
+    srv = Server(chunk_steps=2, slots={(2, 64): 2})
+    stats = srv.run(rs)
+    assert stats["requests"] == 7 and stats["peak_active"] == 2
+    assert sum(res.admitted > min(r.finished for r in srv.results) for res in srv.results) >= 4
+    by_id = {r.rid: r for r in rs}
+    for res in srv.results:
+        r = by_id[res.rid]
+        ref, n = solve_one(r.dim, r.N, r.u_hat, r.t_end)
+        assert res.steps == n, r.rid
+        assert torch.equal(res.u_hat, ref), r.rid
