@@ -498,8 +498,9 @@ bool stage_fused(const azb_solver* s) {
 }
 
 // One evaluation by itself pays for the column stage's idle CUs (129 workgroups at N = 1024)
-// without its gain from the next evaluation's inverse passes: 56 against 55 us FP32 for the
-// separate passes there.
+// without its gain from the next evaluation's inverse passes: 73.7 against 69.6 us FP64 for the
+// separate passes there, 56.4 against 55.5 us FP32.  It concerns single samples: batches of
+// that size have separate passes throughout (stage_shape), and their B_hat anyway.
 bool rhs_alone_separate(int N) { return N == 1024; }
 
 // 2D row kernel over X -> Z, both [component][line][k] with line stride ls, or in column
@@ -1340,7 +1341,9 @@ int azb_autotune_plans(azb_solver* s, const void* u_hat, int reps) {
   if (n == 1) return AZB_OK;
   if (s->dim == 2) {
     // the column stage is built for plan 0; batches that run the separate passes keep it too,
-    // so that they agree with their samples solved alone
+    // so that they agree with their samples solved alone.  That costs them at most 3 % against the
+    // best of the nine pairs of axis-0 plans (us per step: FP32 512^2 x 24 647 against 630, x 8 267
+    // against 262, 1024^2 x 8 990 is the best, FP64 1024^2 x 8 1412 against 1405).
     const int zero[AZB_PROF_FAMILIES] = {};
     return azb_set_plans(s, zero);
   }

@@ -363,7 +363,9 @@ def _used(t: torch.Tensor) -> None:
 
 
 def fft_r2c(u: torch.Tensor) -> torch.Tensor:
-    """Unnormalised R2C over all but the leading (batch) axis."""
+    """Unnormalised R2C over all but the leading (batch) axis.  Queued on the current stream like a
+    torch operation, not waited for: a caller that uses the result on another stream orders
+    the two (``wait_stream``)."""
     _need("fft_r2c", u, (torch.float64, torch.float32),
           lambda sh: 2 <= len(sh) <= 4 and sh[0] >= 1 and len(set(sh[1:])) == 1, "(howmany, n, ..., n)")
     dim = u.dim() - 1
@@ -401,7 +403,8 @@ def _c2r(u_hat: torch.Tensor, n: int, scale: float, overwrite: bool) -> torch.Te
 
 
 def fft_c2r(u_hat: torch.Tensor, n: int) -> torch.Tensor:
-    """Unnormalised C2R; u_hat is left as it is."""
+    """Unnormalised C2R; u_hat is left as it is.  Queued on the current stream, not waited for (see
+    ``fft_r2c``)."""
     _need("fft_c2r", u_hat, (torch.complex128, torch.complex64), _c2r_shape_ok(n),
           _C2R_SHAPE.format(n=n, nh=n // 2 + 1))
     return _c2r(u_hat.resolve_conj().resolve_neg().contiguous(), n, 1.0, False)
@@ -415,7 +418,8 @@ def leray_(u_hat: torch.Tensor) -> torch.Tensor:
 
 
 def initialize(u_phys) -> torch.Tensor:
-    """Initializer::initialize: u_hat = FFT(u) (unnormalised) then Leray, on the device."""
+    """Initializer::initialize: u_hat = FFT(u) (unnormalised) then Leray, on the device.  Queued on the
+    current stream, not waited for (see ``fft_r2c``)."""
     u = torch.as_tensor(u_phys, dtype=torch.float64).to("cuda").contiguous()
     _need("initialize", u, (torch.float64,),
           lambda sh: len(sh) in (3, 4) and sh[0] == len(sh) - 1 and len(set(sh[1:])) == 1 and sh[1] % 2 == 0,
@@ -477,7 +481,8 @@ def to_physical(u_hat: torch.Tensor, N_out: int | None = None) -> torch.Tensor:
     """Velocity in physical space as azeban writes it (run_from_config.cpp:93-98): u_hat
     scaled by 1/N^d, then the unnormalised inverse transform.  With N_out < N the
     spectrum is first truncated to N_out modes per axis, as the sample writer's
-    downsampled output does (netcdf_sample_writer.cpp:143-163); the scale stays 1/N^d."""
+    downsampled output does (netcdf_sample_writer.cpp:143-163); the scale stays 1/N^d.
+    Queued on the current stream, not waited for (see ``fft_r2c``)."""
     dim = u_hat.dim() - 1
     N = u_hat.shape[1]
     n = N if N_out is None else N_out

@@ -106,7 +106,8 @@ int azb_u_max(azb_solver* s, double* u_max_host);
 
 /* One SSP-RK3 step in place on u_hat with dt = min(C/(N u_max(stage 1)), max_dt),
  * SSP_RK3::integrate (include/azeban/evolution/ssp_rk3.hpp:48-64).  dt is taken on
- * the device; dt_host (if not NULL) receives it (synchronising). */
+ * the device; dt_host (if not NULL) receives it (synchronising; refused while the
+ * stream is being captured). */
 int azb_rk3_step(azb_solver* s, void* u_hat, double max_dt, double C, double* dt_host);
 
 /* Simulation::simulate_until (src/azeban/simulation.cpp:89-102): while time < t_end,
@@ -122,7 +123,8 @@ int azb_simulate_until(azb_solver* s, void* u_hat, double t_end, double C, doubl
  * azb_loop_begin sets every sample's time (times0_host[i], or 0 if NULL) and target
  * t_end (synchronising); azb_enqueue_steps queues n steps without synchronising (a
  * step past t_end does nothing on the device, so extra steps are harmless);
- * azb_loop_read copies each sample's time and step count back (synchronising). */
+ * azb_loop_read brings each sample's time and step count back (synchronising; refused
+ * while the stream is being captured, like the reductions below). */
 int azb_loop_begin(azb_solver* s, double t_end, double C, const double* times0_host);
 /* (Re)start one sample of a batched solver without touching the others and without
  * synchronising: queued on the solver's stream, so it takes effect after the steps
