@@ -175,7 +175,7 @@ __global__ void stage_modes_kernel(double2* modes, int N, int nh, double eps, do
 
 // The lines below were placed by timing whole steps (device loop, Fourier states of a
 // shear layer; us per step against the separate passes of the same size, FP64 / FP32).
-// A CU holds one workgroup of 12 waves (148-168 registers), so what counts is the number
+// A CU holds one workgroup of 12 waves (146-168 registers), so what counts is the number
 // of rounds of 256 workgroups and how full the last one is.
 //   N = 64, 128  : width 4, split 2 whatever the batch (N = 64: 57 / 51 against 86 / 101;
 //                  N = 128 x 33: 115 / 84 against 160 / 149)

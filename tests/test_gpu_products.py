@@ -1,7 +1,6 @@
-"""FP64 right-hand sides carry one product less than the oracle: the last diagonal one is
-taken off the others, a gradient that the Leray projection removes mode by mode.  So it
-has to hold for every stored mode, the Nyquist ones and a k_last = 0 plane without
-Hermitian symmetry among them."""
+"""Right-hand sides of white noise in every stored mode, the Nyquist ones and a k_last = 0 plane
+without Hermitian symmetry among them, against the oracle: the divergence of the products and
+its Leray projection hold mode by mode."""
 import math
 
 import numpy as np

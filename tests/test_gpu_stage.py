@@ -28,8 +28,7 @@ def _solver(N, precision):
 
 # batch sizes on both sides of each line of the shape rule: N = 64, 128 have one shape;
 # N = 256 widens its tiles from 8 samples; N = 512 has whole-line tiles at 4 and 13, narrow
-# ones at 2 (FP64: 8 too; FP32 then runs the separate passes); N = 1024 batches are separate,
-# in FP64 only up to two samples
+# ones at 2 (FP64: 8 too; FP32 then runs the separate passes); N = 1024 batches are separate
 @pytest.mark.parametrize("precision", ["fp64", "fp32_mixed"])
 @pytest.mark.parametrize("N,samples", [(64, 3), (128, 2), (256, 7), (256, 8), (512, 2), (512, 4), (512, 8), (512, 13),
                                        (1024, 2), (1024, 3)])
@@ -62,7 +61,7 @@ def test_steps_of_one_call_match_single_steps(cuda, N, precision):
     for _ in range(5):
         t += step.integrate(1e6, max_dt, 0.2, u)
     assert torch.equal(sim.u(), u) and sim.time() == t
-    # a step past the target does nothing, and the last step is clamped onto it
+    # a step past the target does nothing (the clamp within a call: test_gpu_loop_end.py)
     before = sim.u().clone()
     assert sim.simulate_until(sim.time(), chunk=3) == 0 and torch.equal(sim.u(), before)
 
